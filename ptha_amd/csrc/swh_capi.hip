@@ -1367,7 +1367,7 @@ int swh_dispersion_enable(swh_domain *h, double dlon, double dlat, double td1, d
         int rc = dmalloc(&h->dlast, 3 * P);
         if (!rc) rc = dmalloc(&h->drhs, 2 * P);
         for (int k = 0; k < 3 && !rc; k++) rc = dmalloc(&h->dq[k], 2 * P);
-        if (!rc) rc = dmalloc(&h->dwork, 4 * (size_t)h->nx * h->ny * h->esz);
+        if (!rc) rc = dmalloc(&h->dwork, dispersion_work_elems(h->nx, h->ny) * h->esz);
         if (!rc) rc = dmalloc((void **)&h->d_qt, 3 * sizeof(double));
         if (rc) return rc;
         h->disp_on = 1;

@@ -237,7 +237,7 @@ template <typename T>
 hipError_t launch_nonlinear_momentum(const NLArgs<T> &a, bool fused, hipStream_t s);
 
 // Dispersive solve on the staggered grid (swh_dispersion.hip). Planes of pitch * ny
-// except W (4 * nx * ny work for the tridiagonal systems).
+// except W (dispersion_work_elems: the tridiagonal systems).
 template <typename T>
 struct DispArgs {
     int nx, ny, pitch;
@@ -258,6 +258,7 @@ struct DispArgs {
 // from Y0..Y2; then niter tridiagonal iterations (rows of UH, then columns of VH)
 template <typename T>
 hipError_t launch_dispersion(const DispArgs<T> &a, int make_rhs, int extrapolate, int niter, hipStream_t s);
+size_t dispersion_work_elems(int nx, int ny);
 // shift the level times down one and record the new level's time (sc->time or t_host)
 hipError_t launch_dispersion_qt_append(double *qt, const DevScalars *sc, double t_host, hipStream_t s);
 
