@@ -5,10 +5,12 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
 #include "swh_domain.h"
+#include "swh_launch.h"
 
 namespace swh {
 
@@ -1778,8 +1780,11 @@ struct swh_batch {
     long long *d_gidx = nullptr;
     int *d_gij = nullptr;          // the gauges' (i, j), 0-based, for the fused kernel's sampling
     std::vector<int> h_gij;
+    std::map<int, bool> fit_rows;  // gauges_fit_lanes by rows per strip, for these gauges
     double *d_gval = nullptr;      // [slot][sample][3][ng]
-    int block_x = 256, rows_per_block = 32, variant = 2, src_fast = 0;
+    // rows_per_block 0: chosen for each launch from its running sources (batch_rows), at most
+    // rows_most
+    int block_x = 256, rows_per_block = 0, rows_most = 256, variant = 2, src_fast = 0;
     int two_step = 0;              // two fused steps per launch where possible
     int fuse = 2;                  // most fused steps per launch (2..4) where two_step is on
     int xcd_order = 0;             // two-step launches: XCD-aware tile order
@@ -1867,13 +1872,46 @@ int batch_args(swh_batch *b, double dt, LFArgs<T> &a, int &fric_mode)
     return SWH_OK;
 }
 
+// Rows per strip of a launch that takes ns steps of n sources. A strip of r rows walks
+// r + 2 ns - 1 (it recomputes its neighbours'), so tall strips waste least; but the
+// device holds 16 wavefronts per CU of these kernels, and a batch of few sources, or the
+// last ones running of a large one, would leave most of it idle. The time is taken as
+// the rows walked, times the full rounds of resident wavefronts and a share for the last
+// one: a round a quarter, half, three quarters full takes about 0.5, 0.65, 0.85 of a full
+// one (1.42, 1.6, 2.0, 2.33 us a row of five FP32 steps at 1 to 4 wavefronts per SIMD; 1.25,
+// 1.8, 2.5, 2.95 of three FP64 ones). Measured per step against the fixed 256 rows: FP32
+// 1200^2, 1 source 71 -> 7.6 us (16 rows), 3 sources 72 -> 13.6 (24), 12 sources 87 -> 49 (48
+// or 96; 58 at 64, whose second round is nearly empty), 32 sources 129 -> 123; 300^2, 1 source
+// 71 -> 4.7 (8); 512 sources keep the tallest. FP64 against 128 rows: 55 -> 11.3, 66 -> 22, 122
+// -> 99, 260 -> 243 us. Columns per wavefront: 65 - 2 ns (fused), 61 (two steps), 64 lanes of
+// one or four FP32 / two FP64 columns (one step).
+int batch_rows(const swh_batch *b, int n, int ns)
+{
+    if (b->rows_per_block > 0) return b->rows_per_block;
+    const swh_domain *g = b->g;
+    const int vec = (b->variant & 1) ? (g->prec == SWH_PREC_FP64 ? 2 : 4) : 1;
+    const int own = ns == 1 ? 64 * vec : ns == 2 ? 61 : 65 - 2 * ns;
+    const double wx = (double)n * ((g->nx + own - 1) / own), cap = 16.0 * device_cus();
+    static const int rows[] = {256, 192, 128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4};
+    int best = b->rows_most;
+    double cost = 1e300;
+    for (int r : rows) {
+        if (r > b->rows_most) continue;
+        const double w = wx * ((g->ny + r - 1) / r) / cap, q = std::floor(w), rem = w - q;
+        const double last = rem <= 0.0 ? 0.0 : rem <= 0.25 ? 0.5 : rem <= 0.5 ? 0.65 : rem <= 0.75 ? 0.85 : 1.0;
+        const double t = (std::min(r, g->ny) + 2 * ns - 1) * (q + last);
+        if (t < cost) { cost = t; best = r; }
+    }
+    return best;
+}
+
 // One batched step reading buffer c and writing the other.
 template <typename T, bool KAHAN>
 int batch_launch(swh_batch *b, LFArgs<T> &a, int fric_mode, int n_active, int c)
 {
     swh_domain *g = b->g;
     const int o = 1 - c;
-    a.rows_per_block = b->rows_per_block;
+    a.rows_per_block = batch_rows(b, n_active, 1);
     a.src_fast = b->src_fast;
     a.S = (const T *)b->S[c]; a.C = (const T *)b->C[c]; a.UH = (const T *)b->UH[c]; a.VH = (const T *)b->VH[c];
     a.So = (T *)b->S[o]; a.Co = (T *)b->C[o]; a.UHo = (T *)b->UH[o]; a.VHo = (T *)b->VH[o];
@@ -1897,7 +1935,7 @@ int batch_launch2(swh_batch *b, LFArgs<T> &a, int fric_mode, int first, int n, i
 {
     swh_domain *g = b->g;
     const int o = 1 - c;
-    a.rows_per_block = b->rows_per_block;
+    a.rows_per_block = batch_rows(b, n, 2);
     a.src_fast = 0;
     a.src_base = first;
     a.S = (const T *)b->S[c]; a.C = (const T *)b->C[c]; a.UH = (const T *)b->UH[c]; a.VH = (const T *)b->VH[c];
@@ -1913,17 +1951,20 @@ int batch_launch2(swh_batch *b, LFArgs<T> &a, int fric_mode, int first, int n, i
 }
 
 // The fused kernel's lanes hold two gauges each (8-bit indices, 16-bit rows): at most
-// two gauges may share a column within one row strip of the launch shape.
-bool gauges_fit_lanes(const swh_batch *b)
+// two gauges may share a column within one strip of 'rows' rows.
+bool gauges_fit_lanes(swh_batch *b, int rows)
 {
     if (b->ng > 255 || b->g->ny > 65535) return false;
-    const int rows = std::max(1, b->rows_per_block);
+    const auto known = b->fit_rows.find(rows);
+    if (known != b->fit_rows.end()) return known->second;
+    b->fit_rows[rows] = false;
     for (int p = 0; p < b->ng; p++) {
         int same = 0;
         for (int q = 0; q < b->ng; q++)
             same += b->h_gij[2 * q] == b->h_gij[2 * p] && b->h_gij[2 * q + 1] / rows == b->h_gij[2 * p + 1] / rows;
         if (same > 2) return false;
     }
+    b->fit_rows[rows] = true;
     return true;
 }
 
@@ -1936,7 +1977,7 @@ int batch_launchn(swh_batch *b, LFArgs<T> &a, int fric_mode, int first, int n, i
 {
     swh_domain *g = b->g;
     const int o = 1 - c;
-    a.rows_per_block = b->rows_per_block;
+    a.rows_per_block = batch_rows(b, n, ns);
     a.src_fast = 0;
     a.src_base = first;
     a.S = (const T *)b->S[c]; a.C = (const T *)b->C[c]; a.UH = (const T *)b->UH[c]; a.VH = (const T *)b->VH[c];
@@ -1986,9 +2027,10 @@ int batch_evolve(swh_batch *b, double dt, int nsteps)
         // a round of the full depth that every running source takes to its end, the
         // gauge samples inside it written by the launch itself
         int Dg = 0;
-        if (depth >= 3 && gauges_fit_lanes(b)) {
+        if (depth >= 3) {
             Dg = std::min<long long>(depth, nsteps - k);
             while (Dg >= 3 && batch_active(b, b->step + Dg - 1) < n_active) Dg--;
+            if (Dg >= 3 && !gauges_fit_lanes(b, batch_rows(b, n_active, Dg))) Dg = 0;
             // at most one sample inside the round (the launch writes one)
             int due = 0;
             for (int q = 1; q <= Dg; q++) due += sample_due(b, b->step + q) ? 1 : 0;
@@ -2193,12 +2235,13 @@ int swh_batch_create(const swh_domain_desc *desc, int32_t nsources, swh_batch **
     }
     b->nsrc = nsources;
     // default launch: five (FP32) / three (FP64) fused steps per launch, 2-wave blocks,
-    // XCD tile order with sources in groups of 16 (the fastest shapes measured on the
-    // 512-source 1200^2 workload; swh_batch_autotune refines it per batch)
+    // XCD tile order with sources in groups of 16, strips of up to 256 / 128 rows (the fastest
+    // shapes measured on the 512-source 1200^2 workload; shorter strips where a launch has few
+    // sources: batch_rows; swh_batch_autotune refines it per batch)
     b->block_x = 256; b->two_step = 1; b->src_fast = 0;
     b->xcd_order = 1; b->src_group = 16;
-    if (b->g->prec == SWH_PREC_FP64) { b->block_x = 128; b->rows_per_block = 128; b->variant = 3; b->fuse = 3; }
-    else { b->block_x = 128; b->rows_per_block = 256; b->variant = 3; b->fuse = 5; }
+    if (b->g->prec == SWH_PREC_FP64) { b->block_x = 128; b->rows_most = 128; b->variant = 3; b->fuse = 3; }
+    else { b->block_x = 128; b->rows_most = 256; b->variant = 3; b->fuse = 5; }
     const size_t bytes = b->g->plane_elems() * b->g->esz * (size_t)nsources;
     const bool kahan = b->g->prec == SWH_PREC_FP32K;
     for (int k = 0; k < 2 && rc == SWH_OK; k++) {
@@ -2338,6 +2381,7 @@ int swh_batch_gauges_set_schedule(swh_batch *b, int32_t n, const int32_t *ij, in
     if (n > 0) SWH_HIP(hipMemcpy(b->d_gidx, idx.data(), sizeof(long long) * n, hipMemcpyHostToDevice));
     if (n > 0) SWH_HIP(hipMemcpy(b->d_gij, gij.data(), sizeof(int) * 2 * n, hipMemcpyHostToDevice));
     b->h_gij = gij;
+    b->fit_rows.clear();
     b->ng = n; b->gmax = max_samples;
     b->sched.assign(sample_steps, sample_steps + nsamples);
     return SWH_OK;
