@@ -14,6 +14,7 @@
 // The CFL step is a running max of 1/dt kept on the device, so an adaptive rk2 step
 // never returns to the host. Arithmetic follows the reference's evaluation order.
 #include "swh_internal.h"
+#include "swh_lanes.h"
 
 namespace swh {
 
@@ -184,8 +185,7 @@ struct EdgeOut {
     double f0, f1, f2, es_neg, es_pos, mx;
 };
 
-template <typename T>
-__device__ __forceinline__ EdgeOut ns_edge(const FVArgs<T> &a, int j, const Cell &Sc, const Cell &C,
+__device__ __forceinline__ EdgeOut ns_edge(double dbe_j, double inv_cfl, const Cell &Sc, const Cell &C,
                                            const Grad4 &gl, const Grad4 &gc, double e_s, double e_c)
 {
     const double stage_neg = (double)Sc.s + 0.5 * gl.st;
@@ -195,17 +195,16 @@ __device__ __forceinline__ EdgeOut ns_edge(const FVArgs<T> &a, int j, const Cell
     const double u_neg = (double)Sc.u + 0.5 * gl.u, u_pos = (double)C.u - 0.5 * gc.u;
     const double v_neg = (double)Sc.v + 0.5 * gl.v, v_pos = (double)C.v - 0.5 * gc.v;
     const EdgeRes r = edge_flux(stage_neg, stage_pos, depth_neg, depth_pos, u_neg, u_pos, v_neg, v_pos,
-                                (double)Sc.d, (double)C.d, e_s, e_c, a.dbe[j], true);
+                                (double)Sc.d, (double)C.d, e_s, e_c, dbe_j, true);
     EdgeOut o;
     o.f0 = r.f0; o.f1 = r.f1; o.f2 = r.f2;
-    o.es_neg = r.bsp_neg * a.dbe[j] - r.hghh;
-    o.es_pos = 0.0 - r.bsp_pos * a.dbe[j] + r.hghh;
-    o.mx = r.max_speed > 1.0e-12 ? r.max_speed * (1.0 / (a.dle[0] * a.half_cfl)) : 0.0;
+    o.es_neg = r.bsp_neg * dbe_j - r.hghh;
+    o.es_pos = 0.0 - r.bsp_pos * dbe_j + r.hghh;
+    o.mx = r.max_speed > 1.0e-12 ? r.max_speed * inv_cfl : 0.0;
     return o;
 }
 
-template <typename T>
-__device__ __forceinline__ EdgeOut ew_edge(const FVArgs<T> &a, int i, int j, const Cell &Wc, const Cell &C,
+__device__ __forceinline__ EdgeOut ew_edge(double dle_i, double inv_cfl, const Cell &Wc, const Cell &C,
                                            const Grad4 &el, const Grad4 &ec, double e_w, double e_c)
 {
     const double st_neg = (double)Wc.s + 0.5 * el.st;
@@ -215,12 +214,12 @@ __device__ __forceinline__ EdgeOut ew_edge(const FVArgs<T> &a, int i, int j, con
     const double uu_neg = (double)Wc.u + 0.5 * el.u, uu_pos = (double)C.u - 0.5 * ec.u;
     const double vv_neg = (double)Wc.v + 0.5 * el.v, vv_pos = (double)C.v - 0.5 * ec.v;
     const EdgeRes q = edge_flux(st_neg, st_pos, dp_neg, dp_pos, uu_neg, uu_pos, vv_neg, vv_pos, (double)Wc.d,
-                                (double)C.d, e_w, e_c, a.dle[i], false);
+                                (double)C.d, e_w, e_c, dle_i, false);
     EdgeOut o;
     o.f0 = q.f0; o.f1 = q.f1; o.f2 = q.f2;
-    o.es_neg = q.bsp_neg * a.dle[i] - q.hghh;
-    o.es_pos = 0.0 - q.bsp_pos * a.dle[i] + q.hghh;
-    o.mx = q.max_speed > 1.0e-12 ? q.max_speed * (1.0 / (a.dbe[j] * a.half_cfl)) : 0.0;
+    o.es_neg = q.bsp_neg * dle_i - q.hghh;
+    o.es_pos = 0.0 - q.bsp_pos * dle_i + q.hghh;
+    o.mx = q.max_speed > 1.0e-12 ? q.max_speed * inv_cfl : 0.0;
     return o;
 }
 
@@ -232,15 +231,15 @@ __device__ __forceinline__ void cell_sources(const FVArgs<T> &a, int j, const Ce
     if (!a.spherical) return;
     const double half_gravity = 0.5 * kGravity;
     const double dc = (double)C.d;
-    esv = esv + half_gravity * dc * dc * (a.dbe[j + 1] - a.dbe[j]);
+    esv = esv + half_gravity * dc * dc * (scalar_load(a.dbe + j + 1) - scalar_load(a.dbe + j));
     const double uhc = (double)C.uh, vhc = (double)C.vh;
     double cm;
     if (a.coriolis) {
-        cm = a.area[j] * a.cor[j];
+        cm = scalar_load(a.area + j) * scalar_load(a.cor + j);
         esu = esu + cm * vhc;
         esv = esv - cm * uhc;
     }
-    cm = a.area[j] * a.tanlat[j] * (double)C.u;
+    cm = scalar_load(a.area + j) * scalar_load(a.tanlat + j) * (double)C.u;
     esu = esu + cm * vhc;
     esv = esv - cm * uhc;
 }
@@ -258,8 +257,8 @@ __device__ __forceinline__ void cell_sources(const FVArgs<T> &a, int j, const Ce
 // values are loaded one row ahead of their use.
 constexpr int kMOwn = 61;   // owned columns per strip
 
-__device__ __forceinline__ double shfl_from_west(double v) { return __shfl_up(v, 1); }
-__device__ __forceinline__ double shfl_from_east(double v) { return __shfl_down(v, 1); }
+__device__ __forceinline__ double shfl_from_west(double v) { return lane_west(v); }
+__device__ __forceinline__ double shfl_from_east(double v) { return lane_east(v); }
 
 template <typename T>
 __device__ __forceinline__ RawCell<T> raw_clamped(const FVArgs<T> &a, int gi, int j)
@@ -288,6 +287,7 @@ __device__ __forceinline__ void fv_flux_march_body(const FVArgs<T> &a, int rows)
     const bool ew_col = i > 0 && i < a.nx - 1;    // east-west gradients exist in this column
     const Grad4 zero{0.0, 0.0, 0.0, 0.0};
     const long long FP = (long long)a.fpitch * (a.ny + 1), EPn = (long long)a.fpitch * a.ny;
+    const double dle_i = a.dle[gi], inv_ns = 1.0 / (scalar_load(a.dle) * a.half_cfl);   // (the CFL terms' factors)
     // rows j0-2, j0-1, j0 and the north-south gradient of row j0-1
     double e_m2, e_m1, e_0;
     const Cell c_m2 = cell_clamped(a, gi, j0 - 2, e_m2);
@@ -320,12 +320,13 @@ __device__ __forceinline__ void fv_flux_march_body(const FVArgs<T> &a, int rows)
         if (own && j >= 1) {
             const long long o = (long long)j * a.pitch + i;
             const long long fo = (long long)j * a.fpitch + i;
-            const EdgeOut r = ns_edge(a, j, c_m1, c_0, g_prev, g_ns, e_m1, e_0);
+            const double dbe_j = scalar_load(a.dbe + j);
+            const EdgeOut r = ns_edge(dbe_j, inv_ns, c_m1, c_0, g_prev, g_ns, e_m1, e_0);
             a.fNS[fo] = (T)r.f0;
             a.fNS[FP + fo] = (T)r.f1;
             a.fNS[2 * FP + fo] = (T)r.f2;
             a.esJ[fo] = r.es_neg;
-            const EdgeOut q = ew_edge(a, i, j, w, c_0, g_ew_w, g_ew, e_w, e_0);
+            const EdgeOut q = ew_edge(dle_i, 1.0 / (dbe_j * a.half_cfl), w, c_0, g_ew_w, g_ew, e_w, e_0);
             a.fEW[fo] = (T)q.f0;
             a.fEW[EPn + fo] = (T)q.f1;
             a.fEW[2 * EPn + fo] = (T)q.f2;

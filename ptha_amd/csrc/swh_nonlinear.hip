@@ -22,6 +22,7 @@
 // The old UH/VH stay in the current planes and the update writes the spare ones, so
 // the row-carried Coriolis averages of the reference are read directly.
 #include "swh_internal.h"
+#include "swh_lanes.h"
 #include "swh_launch.h"
 
 namespace swh {
@@ -164,7 +165,7 @@ __global__ void nl_flux_kernel(NLArgs<T> a)
         if (i < nx - 1) {
             const int ja = j > 0 ? j - 1 : 0, jb = j;
             const long long qa = (long long)ja * P + i, qb = (long long)jb * P + i;
-            const T dbe = (T)a.dbe[j];
+            const T dbe = (T)scalar_load(a.dbe + j);
             const T vs = VH[qa] + VH[qa + 1];
             const T wa = UVH(i, ja), wb = UVH(i, jb);
             f = dbe * (vs > Z ? wa : wb);
@@ -179,7 +180,7 @@ __global__ void nl_flux_kernel(NLArgs<T> a)
         if (i < nx - 1) {
             const int jm = j > 0 ? j - 1 : 0;
             const long long qm = (long long)jm * P + i;
-            const T dbe = (T)(0.5 * (a.dbe[j] + a.dbe[j + 1]));
+            const T dbe = (T)(0.5 * (scalar_load(a.dbe + j) + scalar_load(a.dbe + j + 1)));
             const T vs = VH[o] + VH[qm];
             const T vm = VVH(i, jm), v0 = VVH(i, j);
             f = dbe * (vs > Z ? vm : v0);
@@ -226,10 +227,10 @@ __global__ void nl_flux_kernel(NLArgs<T> a)
 constexpr int kNLOwn = 61;
 
 template <typename T>
-__device__ __forceinline__ T nl_shl1(T v) { return __shfl_down(v, 1); }   // value of lane + 1
+__device__ __forceinline__ T nl_shl1(T v) { return lane_east(v); }   // value of lane + 1
 
 template <typename T>
-__device__ __forceinline__ T nl_shr1(T v) { return __shfl_up(v, 1); }     // value of lane - 1
+__device__ __forceinline__ T nl_shr1(T v) { return lane_west(v); }   // value of lane - 1
 
 template <typename T>
 struct NLRaw {
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(64) void nl_flux_march_kernel(NLArgs<T> a, int rows
             // NS flux of UH on the bottom edge of row j
             f = Z;
             if (i < nx - 1) {
-                const T dbe = (T)a.dbe[j];
+                const T dbe = (T)scalar_load(a.dbe + j);
                 const T vs = vh_m + vh_me;
                 const T wa = first ? uvh : uvh_m, wb = uvh;
                 f = dbe * (vs > Z ? wa : wb);
@@ -350,7 +351,7 @@ __global__ __launch_bounds__(64) void nl_flux_march_kernel(NLArgs<T> a, int rows
             // NS flux of VH on the bottom edge of row j
             f = Z;
             if (i < nx - 1) {
-                const T dbe = (T)(0.5 * (a.dbe[j] + a.dbe[j + 1]));
+                const T dbe = (T)(0.5 * (scalar_load(a.dbe + j) + scalar_load(a.dbe + j + 1)));
                 const T vs = cur.vh + vh_m;
                 const T vm = first ? vvh : vvh_m, v0 = vvh;
                 f = dbe * (vs > Z ? vm : v0);
