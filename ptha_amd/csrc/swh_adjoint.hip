@@ -13,9 +13,9 @@
 //   pass 2:  lU, lV = identity/Coriolis transpose of (mu = LF*l') + divergence
 //            transpose of lS,
 // each a gather over +-1 neighbours, so no atomics are needed.
-#include <atomic>
 
 #include "swh_internal.h"
+#include "swh_lanes.h"
 #include "swh_launch.h"
 
 namespace swh {
@@ -26,9 +26,9 @@ constexpr int kAdjOwn = 61;   // columns a wavefront writes (lanes 1..61)
 
 // Lane shifts across the wavefront; every lane must execute them.
 template <typename T>
-__device__ __forceinline__ T shl1(T v) { return __shfl_down(v, 1); }   // value of lane + 1
+__device__ __forceinline__ T shl1(T v) { return lane_east(v); }   // value of lane + 1
 template <typename T>
-__device__ __forceinline__ T shr1(T v) { return __shfl_up(v, 1); }     // value of lane - 1
+__device__ __forceinline__ T shr1(T v) { return lane_west(v); }   // value of lane - 1
 
 // h_iph / h_jph of the truely-linear scheme (include.f90:265-280) from the elevations of
 // the two cells of the face (e_far the east or north one)
@@ -63,31 +63,17 @@ struct AdjRow {
     bool mom, in;
 };
 
-// A value that is the same on every lane (a row coefficient), kept in scalar registers
-// so that the three rows carried across iterations take no vector registers.
-__device__ __forceinline__ float uniform(float v)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-__device__ __forceinline__ double uniform(double v)
-{
-    const long long b = __builtin_bit_cast(long long, v);
-    const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffff));
-    const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-
 template <typename T>
 __device__ __forceinline__ AdjRow<T> adj_row(const AdjArgs<T> &a, int r)
 {
     const int rc = min(max(r, 0), a.ny - 1);
     AdjRow<T> q;
-    q.sa = uniform(a.rc.sa[rc]);
-    q.cu = uniform(a.rc.cu[rc]);
-    q.cv = uniform(a.rc.cv[rc]);
-    q.fu = uniform(a.rc.fu[rc]);
-    q.fv = uniform(a.rc.fv[rc]);
-    q.dbe1 = uniform(a.rc.dbe[rc + 1]);
+    q.sa = scalar_load(a.rc.sa + rc);
+    q.cu = scalar_load(a.rc.cu + rc);
+    q.cv = scalar_load(a.rc.cv + rc);
+    q.fu = scalar_load(a.rc.fu + rc);
+    q.fv = scalar_load(a.rc.fv + rc);
+    q.dbe1 = scalar_load(a.rc.dbe + rc + 1);
     q.mom = r >= 0 && r < a.ny - 1;
     q.in = r > 0 && r < a.ny - 1;
     return q;
@@ -120,7 +106,7 @@ __global__ __launch_bounds__(256) void adj_march_kernel(AdjArgs<T> a)
     T lu2 = T(0), lv2 = T(0), hI2 = T(0), hIw2 = T(0), luw2 = T(0), oS2 = T(0), lve2 = T(0), hJ2 = T(0),
       hJe2 = T(0), aV2 = T(0);
     T lv3 = T(0), lve3 = T(0), hJ3 = T(0), hJe3 = T(0);
-    AdjRow<T> q1 = adj_row(a, j0 - 2), q2 = adj_row(a, j0 - 3), q3 = adj_row(a, j0 - 4);
+    AdjRow<T> q1 = adj_row(a, j0 - 2), q2 = adj_row(a, j0 - 3), q3 = adj_row(a, j0 - 4), n_q = adj_row(a, j0 - 1);
 
     // the next two rows' loads are issued before this row is computed (two rows in flight)
     auto load_row = [&](int m, T &ls, T &lu, T &lv, T &e) {
@@ -137,7 +123,8 @@ __global__ __launch_bounds__(256) void adj_march_kernel(AdjArgs<T> a)
         const T ls0 = n_ls, lu0 = n_lu, lv0 = n_lv, e0 = n_e;
         n_ls = nn_ls; n_lu = nn_lu; n_lv = nn_lv; n_e = nn_e;
         if (m + 2 <= j1 + 1) load_row(m + 2, nn_ls, nn_lu, nn_lv, nn_e);
-        const AdjRow<T> q0 = adj_row(a, m);
+        const AdjRow<T> q0 = n_q;
+        n_q = adj_row(a, m + 1);
         const T e0e = shl1(e0);
         // row m: h_iph and aU mu_U (own and the west neighbour's)
         const T hI0 = face_depth(e0, e0e, msl);
@@ -218,11 +205,10 @@ __global__ void adj_inject_kernel(T *lS, int n, const long long *idx, const doub
 template <typename T, bool COR>
 static hipError_t launch_adj_march(const AdjArgs<T> &a0, hipStream_t s)
 {
-    static std::atomic<int> occ[5];
-    constexpr int kBlock = 256;
+    constexpr int kBlock = 64;
     AdjArgs<T> a = a0;
     if (a.rows <= 0)
-        a.rows = occupancy_rows((const void *)adj_march_kernel<T, COR>, occ, a.nx, a.ny, kBlock, kAdjOwn, 3);
+        a.rows = fused_rows(a.nx, a.ny, 1, 2, kAdjOwn, 256);
     const int waves = (a.nx + kAdjOwn - 1) / kAdjOwn, wpb = kBlock / 64;
     dim3 grid((waves + wpb - 1) / wpb, (a.ny + a.rows - 1) / a.rows);
     hipLaunchKernelGGL((adj_march_kernel<T, COR>), grid, dim3(kBlock), 0, s, a);

@@ -156,4 +156,92 @@ __device__ void bf_lines(const BfLines &b, int nx, int ny, int pitch, const T *_
     sc->time = t;
 }
 
+// The sums of bf_lines from line buffers [level][side N, E, S, W][len] (the pre-step UH/VH of
+// 'levels' steps that an earlier launch took, at most kBfLevels), by nlb workgroups of
+// which this is the k'th: the same split of a side over its workgroups, the same trees and
+// the same bookkeeping, step by step.
+constexpr int kBfLevels = 6;
+
+template <typename T>
+__device__ void bf_sum_lines(const BfLines &b, int nx, int ny, const T *__restrict__ lines, int len_max, int levels,
+                             int k, int nlb)
+{
+    const int ne = b.n_ext;
+    const int q = k & 3, r = k >> 2, nbq = (nlb - q + 3) >> 2;
+    const int len = max((q & 1) == 0 ? nx - 2 * ne : ny - 2 * ne, 0);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    __shared__ double wsum[4][kBfLevels][2];
+    __shared__ double st[kBfLevels][4];
+    __shared__ int last;
+    for (int l = 0; l < levels; l++) {
+        const T *__restrict__ p = lines + (4 * l + q) * len_max;
+        DD x{0.0, 0.0};
+        for (int c = r * blockDim.x + threadIdx.x; c < len; c += nbq * blockDim.x) x = dd_add(x, (double)p[c]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const DD y{__shfl_down(x.hi, off), __shfl_down(x.lo, off)};
+            x = dd_add(x, y);
+        }
+        if (lane == 0) {
+            wsum[w][l][0] = x.hi;
+            wsum[w][l][1] = x.lo;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double *part = b.part + (size_t)k * (2 * kBfLevels);
+        for (int l = 0; l < levels; l++) {
+            DD x{wsum[0][l][0], wsum[0][l][1]};
+            for (int ww = 1; ww < nw; ww++) x = dd_add(x, DD{wsum[ww][l][0], wsum[ww][l][1]});
+            __hip_atomic_store(part + 2 * l, x.hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(part + 2 * l + 1, x.lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        // (ordering as in bf_lines)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const unsigned int done =
+            __hip_atomic_fetch_add(&b.sc->bf_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = done == (unsigned int)(nlb - 1);
+        if (last) __hip_atomic_store(&b.sc->bf_done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!last) return;
+    for (int pair = w; pair < 4 * levels; pair += nw) {
+        const int qq = pair & 3, ll = pair >> 2;
+        const int nb = (nlb - qq + 3) >> 2;
+        DD x{0.0, 0.0};
+        for (int rr = lane; rr < nb; rr += 64) {
+            const double *p = b.part + (size_t)(qq + 4 * rr) * (2 * kBfLevels) + 2 * ll;
+            const double hi = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const double lo = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            x = dd_add(x, DD{hi, lo});
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            const DD y{__shfl_down(x.hi, off), __shfl_down(x.lo, off)};
+            x = dd_add(x, y);
+        }
+        if (lane == 0) st[ll][qq] = x.hi + x.lo;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    DevScalars *sc = b.sc;
+    const double m0 = b.dbe[ny - ne], m1 = b.dle[nx - ne], m2 = b.dbe[ne], m3 = b.dle[ne];
+    double t = sc->time, bf_time = sc->bf_time, ev = 0.0, b0 = 0.0, b1 = 0.0, b2 = 0.0, b3 = 0.0;
+    for (int l = 0; l < levels; l++) {
+        b0 = st[l][0] * m0;
+        b1 = st[l][1] * m1;
+        b2 = -st[l][2] * m2;
+        b3 = -st[l][3] * m3;
+        ev = (((b0 + b1) + b2) + b3) * b.dt;
+        bf_time = bf_time + ev;
+        t = b.t_after[l];
+    }
+    sc->bf_store[0] = b0;
+    sc->bf_store[1] = b1;
+    sc->bf_store[2] = b2;
+    sc->bf_store[3] = b3;
+    sc->bf_evolve = ev;
+    sc->bf_time = bf_time;
+    sc->time = t;
+}
+
 }  // namespace swh

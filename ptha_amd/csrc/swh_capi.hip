@@ -510,6 +510,165 @@ int leapfrog_step2(swh_domain *h, double dt, bool mid_sample = false)
     return SWH_OK;
 }
 
+// At most two of n gauges (0-based (i, j) pairs) share a column within one strip of 'rows'
+// rows: what the lanes of the fused kernel hold (8-bit indices, 16-bit rows).
+bool gauges_fit(const std::vector<int> &ij, int n, int ny, int rows)
+{
+    if (n > 255 || ny > 65535 || rows < 1) return false;
+    for (int p = 0; p < n; p++) {
+        int same = 0;
+        for (int q = 0; q < n; q++)
+            same += ij[2 * q] == ij[2 * p] && ij[2 * q + 1] / rows == ij[2 * p + 1] / rows;
+        if (same > 2) return false;
+    }
+    return true;
+}
+
+bool gauges_fit_rows(swh_domain *h, int rows)
+{
+    const auto known = h->fit_rows.find(rows);
+    if (known != h->fit_rows.end()) return known->second;
+    return h->fit_rows[rows] = gauges_fit(h->h_gij, h->ng, h->ny, rows);
+}
+
+// The boundary-flux sums that the last fused launch of a call has left to a following one.
+int bf_flush(swh_domain *h)
+{
+    if (!h->lb_pending) return SWH_OK;
+    BfLines b = bf_args(h, 256, h->lb_dt, 0.0, 0.0);
+    for (int l = 0; l < h->lb_pending; l++) b.t_after[l] = h->lb_t[l];
+    const size_t off = (size_t)(1 - h->lb_cur) * 24 * h->lb_len;
+    const int levels = h->lb_pending;
+    h->lb_pending = 0;
+    if (h->prec == SWH_PREC_FP64)
+        SWH_HIP(launch_bf_flush<double>(b, h->nx, h->ny, (const double *)h->d_lb + off, h->lb_len, levels, h->stream));
+    else
+        SWH_HIP(launch_bf_flush<float>(b, h->nx, h->ny, (const float *)h->d_lb + off, h->lb_len, levels, h->stream));
+    return SWH_OK;
+}
+
+// how many of the next ns steps update max_U
+int maxq_due(const swh_domain *h, int ns)
+{
+    int due = 0;
+    if (h->maxq_mask)
+        for (int k = 0; k < ns; k++) due += (h->nsteps + k) % h->maxq_freq == 0;
+    return due;
+}
+
+// Whether the next ns leapfrog steps can run as one fused launch: as two_step_ok, for ns
+// steps, and max_U not due in any of them, or max_stage alone due in all (which the launch
+// keeps; a mixture would need its masks in the loop).
+bool fused_ok(const swh_domain *h, double dt, int ns)
+{
+    if (!h->two_step || h->rows2 || !h->d_lb || h->bc_mask || h->n_nest_strips ||
+        h->nx <= 2 * h->n_ext || h->ny <= 2 * h->n_ext)
+        return false;
+    if (h->method == SWH_METHOD_LLPNF && (!h->truely_linear || !h->fw_ready)) return false;
+    if (h->f_on) {
+        double t = h->time;
+        for (int k = 0; k < ns; k++) {
+            const double t_half = t + dt * 0.5;
+            if (forcing_fraction(h, t_half, dt) != 0.0) return false;
+            t = t_half + 0.5 * dt;
+        }
+    }
+    const int due = maxq_due(h, ns);
+    if (due && (due != ns || h->maxq_mask != SWH_MAXQ_MAX_STAGE)) return false;
+    return (long long)h->pitch * h->ny < (1LL << 31);
+}
+
+// Steps of the next fused launch with 'left' steps to go (0: take a step or a pair
+// another way): three where the rest divides by three, so that what is left over goes first
+// and the last launch's sums are the only ones flushed. Deeper launches move less memory, but
+// walk more rows per strip: four or five FP32 steps take 5.8-7.1 us a step against 5.6 at
+// 1024^2, 3.9-4.3 against 3.4 at 400^2, and 11.9-13.2 against 12.7 at 2048^2.
+int fused_depth(long long left)
+{
+    return left % 3 == 0 && left > 0 ? 3 : 0;
+}
+
+int fused_strip_rows(const swh_domain *h, int ns)
+{
+    return fused_rows(h->nx, h->ny, 1, ns, 65 - 2 * ns, h->prec == SWH_PREC_FP64 ? 128 : 256);
+}
+
+// ns leapfrog steps in one launch (swh_leapfrog_sg.hip). level (1..ns, or 0): also record
+// a gauge sample after that step.
+template <typename T, bool KAHAN>
+int leapfrog_fused(swh_domain *h, double dt, int ns, int level = 0)
+{
+    if (h->rc_dt != dt) {
+        int rc = build_rc<T>(h, dt);
+        if (rc) return rc;
+    }
+    if (h->nsteps == 0) {
+        int rc = maxq_now<T>(h, nullptr, h->time);
+        if (rc) return rc;
+    }
+    const int c = h->cur, o = 1 - c, fric_mode = h->method == SWH_METHOD_LLPNF ? 1 : 0;
+    LFArgs<T> a;
+    a.nx = h->nx; a.ny = h->ny; a.pitch = h->pitch; a.src_stride = 0;
+    a.S = (const T *)h->S[c]; a.C = (const T *)h->C[c]; a.UH = (const T *)h->UH[c]; a.VH = (const T *)h->VH[c];
+    a.E = (const T *)h->E;
+    a.So = (T *)h->S[o]; a.Co = (T *)h->C[o]; a.UHo = (T *)h->UH[o]; a.VHo = (T *)h->VH[o];
+    a.rc = rc_view<T>(h);
+    a.fwU = (const T *)h->fwU; a.fwV = (const T *)h->fwV; a.nsq = nullptr;
+    a.msl = (T)h->msl; a.dt = (T)dt; a.dt_lfc = (T)(dt * h->lfc);
+    a.lin_fric_mult = (T)(1.0 / (1.0 + dt * h->lfc));
+    a.fric_power = T(0);
+    a.bc_mask = 0; a.bc_stage = T(0);
+    a.rows_per_block = fused_strip_rows(h, ns);
+    a.src_fast = 0;
+    a.maxq_mask = 0; a.mx = (T *)h->mx; a.t_after = T(0); a.arrival_stage = T(0);
+    a.lf2_order = 1; a.lf2_group = 1;
+    if (maxq_due(h, ns)) a.mx_levels = (1 << ns) - 1;
+    // the boundary fluxes: this launch's lines into one buffer, the sums of the launch before
+    // it from the other
+    const size_t half = (size_t)24 * h->lb_len;
+    a.lb_len = h->lb_len;
+    a.lb_out = (T *)h->d_lb + h->lb_cur * half;
+    a.bf.n_ext = h->n_ext;
+    if (h->lb_pending) {
+        a.bf = bf_args(h, 128, h->lb_dt, 0.0, 0.0);
+        for (int l = 0; l < h->lb_pending; l++) a.bf.t_after[l] = h->lb_t[l];
+        a.lb_in = (const T *)h->d_lb + (1 - h->lb_cur) * half;
+        a.lb_levels = h->lb_pending;
+    }
+    double t = h->time, t_prev = t, ends[6];
+    for (int k = 0; k < ns; k++) {
+        t_prev = t;
+        t = (t + dt * 0.5) + 0.5 * dt;
+        ends[k] = t;
+    }
+    if (level) {
+        if (!h->d_gij || h->ng < 1) return fail(SWH_ESTATE, "gauges not set");
+        if (h->gsamples >= h->gmax) return fail(SWH_ESTATE, "gauge sample buffer full");
+        a.g_n = h->ng; a.g_max = h->gmax; a.g_ij = h->d_gij; a.g_val = h->d_gval;
+        a.g_level = level; a.g_sample = h->gsamples;
+        a.g_time = h->d_gtime + h->gsamples;
+        a.g_t = ends[level - 1];
+    }
+    SWH_HIP(launch_leapfrog_sg<T, KAHAN>(a, h->coriolis, fric_mode, h->truely_linear, h->lfc != 0.0, ns, h->stream));
+    if (level) h->gsamples++;
+    for (int k = 0; k < ns; k++) h->lb_t[k] = ends[k];
+    h->lb_pending = ns;
+    h->lb_dt = dt;
+    h->lb_cur = 1 - h->lb_cur;
+    h->cur = o;
+    h->time = t;
+    h->dt_last_update = dt;
+    h->evolve_step_dt = t - t_prev;
+    h->nsteps += ns;
+    return SWH_OK;
+}
+
+int leapfrog_fused_any(swh_domain *h, double dt, int ns, int level = 0)
+{
+    return h->prec == SWH_PREC_FP64 ? leapfrog_fused<double, false>(h, dt, ns, level)
+                                    : leapfrog_fused<float, true>(h, dt, ns, level);
+}
+
 template <typename T>
 FVArgs<T> fv_args(swh_domain *h, int dst, int src)
 {
@@ -717,6 +876,30 @@ int evolve(swh_domain *h, double dt)
 }  // namespace
 
 namespace swh {
+
+// A strip of r rows walks r + 2 ns - 1 (it recomputes its neighbours'; two per iteration of
+// the loop, so odd r waste nothing): tall strips waste least, but leave the device idle on a
+// single grid, in a batch of few sources, or by the last ones running of a large one. The time
+// of a launch is that of the rows walked; a row takes longer the more wavefronts a SIMD has:
+// 0.55 + 0.24 n us for n of them (1 and more) in a launch of three FP32 steps, 0.75 + 0.39 n
+// in FP64, 1.1 + 0.41 n in one of five FP32 steps: close to 2.3 + n in all of them. Measured per
+// step with max_stage, in us, for 3 / 5 / 9 / 15 / 23 / 47 rows a strip: 400^2 FP64 4.5 / 5.3 /
+// 6.2 / 8.6 / 11.9 / 21.4; 2048^2 FP32 18.9 / 15.6 / 15.3 / 15.0 / 16.3 / 22.2; 12 sources of
+// 1200^2 in FP32, five steps: 99 / 71 / 53 / 45 / 43 / 43 (78 at 255); 32 sources: 257 / 184 /
+// 137 / 115 / 105 / 100 (123). Strips of three rows with five steps lose to the model's
+// count (300^2, 1 source: 3.6, 3.3 with five rows), hence the least height.
+int fused_rows(int nx, int ny, int n, int ns, int own, int most)
+{
+    const double wx = (double)n * ((nx + own - 1) / own) / (4.0 * device_cus());
+    int best = most;
+    double cost = 1e300;
+    for (int r = most - 1; r >= (ns > 3 ? 5 : 3); r -= r > 127 ? 16 : r > 31 ? 4 : 2) {
+        const int walked = (std::min(r, ny) + 2 * ns) & ~1;
+        const double t = walked * (2.3 + std::max(1.0, wx * ((ny + r - 1) / r)));
+        if (t < cost) { cost = t; best = r; }
+    }
+    return best;
+}
 
 int domain_evolve(swh_domain *h, double dt) { return evolve(h, dt); }
 
@@ -934,7 +1117,11 @@ int swh_domain_create(const swh_domain_desc *d, swh_domain **out)
     // line workgroups: at most 4 ceil(max(nx, ny) / 64) wanted, in rows at most
     // ceil(nx / 64) workgroups wide
     h->bf_cap = 4 * ((std::max(nx, ny) + 63) / 64) + (nx + 63) / 64;
-    A((void **)&h->d_bfpart, sizeof(double) * 4 * (size_t)h->bf_cap);
+    A((void **)&h->d_bfpart, sizeof(double) * 12 * (size_t)h->bf_cap);
+    if (h->method == SWH_METHOD_LINEAR || h->method == SWH_METHOD_LLPNF) {
+        h->lb_len = std::max(nx, ny) - 2 * n_ext;
+        A(&h->d_lb, (size_t)2 * 6 * 4 * h->lb_len * h->esz);
+    }
     A((void **)&h->d_work, sizeof(double) * (2 * (size_t)ny + 16));
     if (rc) {
         swh_domain_destroy(h);
@@ -979,7 +1166,7 @@ int swh_domain_destroy(swh_domain *h)
                     h->d_gval, h->d_gtime, h->adj[0][0], h->adj[0][1], h->adj[0][2], h->adj[1][0],
                     h->adj[1][1], h->adj[1][2], h->d_gvec, h->d_bmax, h->d_bfpart, h->fS, h->fUH, h->fVH, h->fE,
                     h->nlw, h->d_corbe, h->dlast, h->drhs, h->dq[0], h->dq[1], h->dq[2], h->dwork, h->d_qt,
-                    h->d_stats, h->d_ggrad, h->ring, h->d_stage};
+                    h->d_stats, h->d_ggrad, h->ring, h->d_stage, h->d_lb, h->d_gij};
     for (void *p : ptrs) dfree(p);
     for (void *p : h->ckpt) dfree(p);
     dfree(h->snap);
@@ -1128,6 +1315,18 @@ int swh_evolve_steps(swh_domain *h, double timestep, int32_t nsteps)
     if (nsteps < 0) return fail(SWH_EINVAL, "nsteps must be >= 0");
     for (int k = 0; k < nsteps;) {
         int rc;
+        const int ns = timestep > 0.0 && h->d_lb ? fused_depth(nsteps - k) : 0;
+        if (ns && fused_ok(h, timestep, ns)) {
+            rc = leapfrog_fused_any(h, timestep, ns);
+            k += ns;
+            if (!rc && k >= nsteps) rc = bf_flush(h);
+            if (rc) {
+                h->lb_pending = 0;
+                return rc;
+            }
+            continue;
+        }
+        if ((rc = bf_flush(h))) return rc;
         if (k + 1 < nsteps && timestep > 0.0 && two_step_ok(h, timestep)) {
             rc = h->prec == SWH_PREC_FP64 ? leapfrog_step2<double, false>(h, timestep)
                                           : leapfrog_step2<float, true>(h, timestep);
@@ -1313,14 +1512,19 @@ int swh_gauges_set(swh_domain *h, int32_t n, const int32_t *ij, int32_t max_samp
         idx[g] = (long long)j * h->pitch + i;
     }
     SWH_HIP(hipStreamSynchronize(h->stream));
-    dfree(h->d_gidx); dfree(h->d_gval); dfree(h->d_gtime);
-    h->d_gidx = nullptr; h->d_gval = nullptr; h->d_gtime = nullptr;
+    dfree(h->d_gidx); dfree(h->d_gval); dfree(h->d_gtime); dfree(h->d_gij);
+    h->d_gidx = nullptr; h->d_gval = nullptr; h->d_gtime = nullptr; h->d_gij = nullptr;
+    h->h_gij.resize(2 * (size_t)n);
+    for (int k = 0; k < 2 * n; k++) h->h_gij[k] = ij[k] - 1;
     int rc = dmalloc((void **)&h->d_gidx, sizeof(long long) * (n > 0 ? n : 1));
+    if (!rc) rc = dmalloc((void **)&h->d_gij, sizeof(int) * 2 * (n > 0 ? n : 1));
     if (!rc) rc = dmalloc((void **)&h->d_gval, sizeof(double) * 3 * (size_t)(n > 0 ? n : 1) * max_samples);
     if (!rc) rc = dmalloc((void **)&h->d_gtime, sizeof(double) * max_samples);
     if (rc) return rc;
     if (n > 0) SWH_HIP(hipMemcpy(h->d_gidx, idx.data(), sizeof(long long) * n, hipMemcpyHostToDevice));
+    if (n > 0) SWH_HIP(hipMemcpy(h->d_gij, h->h_gij.data(), sizeof(int) * 2 * n, hipMemcpyHostToDevice));
     h->ng = n; h->gmax = max_samples; h->gsamples = 0;
+    h->fit_rows.clear();
     return SWH_OK;
 }
 
@@ -1629,7 +1833,37 @@ int swh_evolve_record_gauges_schedule(swh_domain *h, double timestep, int32_t ns
         rc = swh_gauges_sample(h);
         q = 1;
     }
+    // fused launches take one sample inside where the scheme allows (truely-linear 'linear',
+    // gauges that fit the lanes), else they end at it
+    const bool inside = h->method == SWH_METHOD_LINEAR && h->truely_linear && h->ng > 0 && h->d_gij;
     while (!rc && n < last) {
+        int ns = h->d_lb ? fused_depth(last - n) : 0;
+        if (ns) {
+            const auto count = [&](int m) {   // samples due in the next m steps
+                int due = 0;
+                while (q + due < nsamples && sample_steps[q + due] <= n + m) due++;
+                return due;
+            };
+            if (ns == 5 && count(5) > 1) ns = 3;
+            const int due = count(ns);
+            int level = due ? (int)(sample_steps[q] - n) : 0;
+            const bool at_end = due == 1 && level == ns;
+            if (due && !(due == 1 && inside && !maxq_due(h, ns) && gauges_fit_rows(h, fused_strip_rows(h, ns)))) {
+                if (!at_end) ns = 0;
+                level = 0;
+            }
+            if (ns && fused_ok(h, timestep, ns)) {
+                rc = leapfrog_fused_any(h, timestep, ns, level);
+                n += ns;
+                if (level) q++;
+                if (!rc && q < nsamples && sample_steps[q] == n) {
+                    rc = swh_gauges_sample(h);
+                    q++;
+                }
+                continue;
+            }
+        }
+        if ((rc = bf_flush(h))) break;
         const bool mid = q < nsamples && sample_steps[q] == n + 1;
         if (n + 2 <= last && two_step_ok(h, timestep) && (!mid || h->ng > 0)) {
             rc = h->prec == SWH_PREC_FP64 ? leapfrog_step2<double, false>(h, timestep, mid)
@@ -1645,6 +1879,8 @@ int swh_evolve_record_gauges_schedule(swh_domain *h, double timestep, int32_t ns
             q++;
         }
     }
+    if (!rc) rc = bf_flush(h);
+    h->lb_pending = 0;
     return rc;
 }
 
@@ -1872,37 +2108,28 @@ int batch_args(swh_batch *b, double dt, LFArgs<T> &a, int &fric_mode)
     return SWH_OK;
 }
 
-// Rows per strip of a launch that takes ns steps of n sources. A strip of r rows walks
-// r + 2 ns - 1 (it recomputes its neighbours'), so tall strips waste least; but the
-// device holds 16 wavefronts per CU of these kernels, and a batch of few sources, or the
-// last ones running of a large one, would leave most of it idle. The time is taken as
-// the rows walked, times the full rounds of resident wavefronts and a share for the last
-// one: a round a quarter, half, three quarters full takes about 0.5, 0.65, 0.85 of a full
-// one (1.42, 1.6, 2.0, 2.33 us a row of five FP32 steps at 1 to 4 wavefronts per SIMD; 1.25,
-// 1.8, 2.5, 2.95 of three FP64 ones). Measured per step against the fixed 256 rows: FP32
-// 1200^2, 1 source 71 -> 7.6 us (16 rows), 3 sources 72 -> 13.6 (24), 12 sources 87 -> 49 (48
-// or 96; 58 at 64, whose second round is nearly empty), 32 sources 129 -> 123; 300^2, 1 source
-// 71 -> 4.7 (8); 512 sources keep the tallest. FP64 against 128 rows: 55 -> 11.3, 66 -> 22, 122
-// -> 99, 260 -> 243 us. Columns per wavefront: 65 - 2 ns (fused), 61 (two steps), 64 lanes of
-// one or four FP32 / two FP64 columns (one step).
+// Rows per strip of a launch that takes ns steps of n sources (fused_rows); columns per
+// wavefront: 65 - 2 ns (fused), 61 (two steps), 64 lanes of one or four FP32 / two FP64
+// columns (one step).
 int batch_rows(const swh_batch *b, int n, int ns)
 {
     if (b->rows_per_block > 0) return b->rows_per_block;
     const swh_domain *g = b->g;
     const int vec = (b->variant & 1) ? (g->prec == SWH_PREC_FP64 ? 2 : 4) : 1;
     const int own = ns == 1 ? 64 * vec : ns == 2 ? 61 : 65 - 2 * ns;
-    const double wx = (double)n * ((g->nx + own - 1) / own), cap = 16.0 * device_cus();
-    static const int rows[] = {256, 192, 128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4};
-    int best = b->rows_most;
-    double cost = 1e300;
-    for (int r : rows) {
-        if (r > b->rows_most) continue;
-        const double w = wx * ((g->ny + r - 1) / r) / cap, q = std::floor(w), rem = w - q;
-        const double last = rem <= 0.0 ? 0.0 : rem <= 0.25 ? 0.5 : rem <= 0.5 ? 0.65 : rem <= 0.75 ? 0.85 : 1.0;
-        const double t = (std::min(r, g->ny) + 2 * ns - 1) * (q + last);
-        if (t < cost) { cost = t; best = r; }
-    }
-    return best;
+    return fused_rows(g->nx, g->ny, n, ns, own, b->rows_most);
+}
+
+// Most steps of a launch over n running sources. Deeper launches move less memory per step,
+// which counts once the launch fills the device; below that the rows that their strips
+// recompute cost more. FP32 us per step, three / five steps: 3 sources of 1200^2 10.1 / 13.1,
+// 6 sources 25.9 / 22.9, 24 of 300^2 7.4 / 8.9; FP64, three / four: 3 sources 13.8 / 16.7, 6
+// 37.6 / 35.5, 32 184 / 153.
+int batch_depth(const swh_batch *b, int n)
+{
+    if (b->rows_per_block > 0) return b->fuse;   // a shape that was set or tuned
+    const bool full = (double)n * b->g->nx * b->g->ny > 6e6;
+    return b->g->prec == SWH_PREC_FP64 ? (full ? 4 : 3) : (full ? 5 : 3);
 }
 
 // One batched step reading buffer c and writing the other.
@@ -1950,22 +2177,12 @@ int batch_launch2(swh_batch *b, LFArgs<T> &a, int fric_mode, int first, int n, i
     return SWH_OK;
 }
 
-// The fused kernel's lanes hold two gauges each (8-bit indices, 16-bit rows): at most
-// two gauges may share a column within one strip of 'rows' rows.
+// gauges_fit for this batch's gauges and strips of 'rows' rows
 bool gauges_fit_lanes(swh_batch *b, int rows)
 {
-    if (b->ng > 255 || b->g->ny > 65535) return false;
     const auto known = b->fit_rows.find(rows);
     if (known != b->fit_rows.end()) return known->second;
-    b->fit_rows[rows] = false;
-    for (int p = 0; p < b->ng; p++) {
-        int same = 0;
-        for (int q = 0; q < b->ng; q++)
-            same += b->h_gij[2 * q] == b->h_gij[2 * p] && b->h_gij[2 * q + 1] / rows == b->h_gij[2 * p + 1] / rows;
-        if (same > 2) return false;
-    }
-    b->fit_rows[rows] = true;
-    return true;
+    return b->fit_rows[rows] = gauges_fit(b->h_gij, b->ng, b->g->ny, rows);
 }
 
 // One launch advancing slots [first, first + n) by ns (3 to 6) steps (reads buffer c);
@@ -1978,6 +2195,9 @@ int batch_launchn(swh_batch *b, LFArgs<T> &a, int fric_mode, int first, int n, i
     swh_domain *g = b->g;
     const int o = 1 - c;
     a.rows_per_block = batch_rows(b, n, ns);
+    // (few sources: one wavefront per workgroup leaves none idle past the east edge; 3 sources
+    // of 1200^2 10.1 against 11.2 us a step, 8 of 300^2 4.4 against 4.6)
+    const int bx = b->rows_per_block > 0 || ns > 3 ? b->block_x : 64;
     a.src_fast = 0;
     a.src_base = first;
     a.S = (const T *)b->S[c]; a.C = (const T *)b->C[c]; a.UH = (const T *)b->UH[c]; a.VH = (const T *)b->VH[c];
@@ -1995,7 +2215,7 @@ int batch_launchn(swh_batch *b, LFArgs<T> &a, int fric_mode, int first, int n, i
             }
     }
     const hipError_t e = launch_leapfrogn<T, KAHAN>(a, g->coriolis, fric_mode, g->truely_linear, g->lfc != 0.0, n,
-                                                    b->block_x, g->stream, (b->variant & 2) ? 1 : 0, ns);
+                                                    bx, g->stream, (b->variant & 2) ? 1 : 0, ns);
     a.g_n = 0; a.g_level = 0;
     SWH_HIP(e);
     b->n_launch++; b->src_launch += n; b->src_steps += (long long)ns * n;
@@ -2016,10 +2236,10 @@ int batch_evolve(swh_batch *b, double dt, int nsteps)
         if (rc) return rc;
     }
     const bool can2 = b->two_step && fric_mode <= 1 && (long long)b->g->plane_elems() < (1LL << 31);
-    const int depth = can2 ? std::max(2, std::min(6, b->fuse)) : 1;   // most steps per launch
     for (int k = 0; k < nsteps;) {
         const int n_active = batch_active(b, b->step);
         if (n_active == 0) break;
+        const int depth = can2 ? std::max(2, std::min(6, batch_depth(b, n_active))) : 1;   // most steps per launch
         const int c = b->cur, o = 1 - c;
         const bool sample_next = sample_due(b, b->step + 1);
         int n_last;   // sources that took the last step of this round
@@ -2121,7 +2341,7 @@ int batch_evolve(swh_batch *b, double dt, int nsteps)
 // writes the other, which the next real step overwrites), so the state and step count
 // are unchanged. One-step shapes: variant 0..15 x block_x {64,128,256} x rows
 // {16,32,64}; then the fused kernels: 2..5 steps per launch x block_x x rows
-// {32,...,256} x tile order (hardware, or XCD order with sources interleaved in groups
+// {31,...,255} x tile order (hardware, or XCD order with sources interleaved in groups
 // of 16), compared per cell-update of the running sources.
 template <typename T, bool KAHAN>
 int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *best_ms)
@@ -2177,7 +2397,7 @@ int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *bes
         const int v1 = bv | 2;
         b->variant = v1 & 7; b->src_fast = (v1 >> 3) & 1;
         const int orders[2][2] = {{0, 1}, {1, 16}};
-        const int rws[4] = {32, 64, 128, 256};
+        const int rws[4] = {31, 63, 127, 255};   // (the loop takes rows in pairs: fused_rows)
         for (int D = 2; D <= 5 && rc == SWH_OK; D++)
             for (int io = 0; io < 2 && rc == SWH_OK; io++)
                 for (int ib = 0; ib < 3 && rc == SWH_OK; ib++)
@@ -2234,10 +2454,10 @@ int swh_batch_create(const swh_domain_desc *desc, int32_t nsources, swh_batch **
         return rc;
     }
     b->nsrc = nsources;
-    // default launch: five (FP32) / three (FP64) fused steps per launch, 2-wave blocks,
-    // XCD tile order with sources in groups of 16, strips of up to 256 / 128 rows (the fastest
-    // shapes measured on the 512-source 1200^2 workload; shorter strips where a launch has few
-    // sources: batch_rows; swh_batch_autotune refines it per batch)
+    // default launch: fused steps (batch_depth), 2-wave blocks, XCD tile order with sources in
+    // groups of 16, strips of up to 256 / 128 rows (the fastest shapes measured on the
+    // 512-source 1200^2 workload; shorter strips where a launch has few sources: batch_rows;
+    // swh_batch_autotune refines it per batch)
     b->block_x = 256; b->two_step = 1; b->src_fast = 0;
     b->xcd_order = 1; b->src_group = 16;
     if (b->g->prec == SWH_PREC_FP64) { b->block_x = 128; b->rows_most = 128; b->variant = 3; b->fuse = 3; }

@@ -1,5 +1,6 @@
 // The device-side state of one SWALS domain (shared by the C ABI translation units).
 #pragma once
+#include <map>
 #include <vector>
 
 #include "swh_internal.h"
@@ -95,10 +96,19 @@ struct swh_domain {
     // them): rows per strip of that kernel (0: chosen from its occupancy) and threads
     // per workgroup
     int two_step = 1, rows2 = 0, block2 = 256;
-    // partial sums of the boundary-flux line workgroups of the step launches (16
+    // partial sums of the boundary-flux line workgroups of the step launches (12
     // doubles per workgroup, room for bf_cap of them)
     double *d_bfpart = nullptr;
     int bf_cap = 0;
+    // fused launches of several steps: UH/VH on the boundary-flux lines, two buffers of 6
+    // levels x 4 sides x lb_len in turn (d_lb); lb_pending levels of buffer lb_cur, whose steps
+    // ended at lb_t, are still to be summed (within a call only: bf_flush ends it)
+    void *d_lb = nullptr;
+    int lb_len = 0, lb_cur = 0, lb_pending = 0;
+    double lb_t[6] = {}, lb_dt = 0.0;
+    int *d_gij = nullptr;          // the gauges' (i, j), 0-based
+    std::vector<int> h_gij;
+    std::map<int, bool> fit_rows;  // whether they fit the fused kernel's lanes, by rows per strip
 
     // staggered leapfrog family (time kept on the host, fixed timestep)
     bool leapfrog() const

@@ -57,7 +57,7 @@ struct DevScalars {
 // Boundary-flux sums of a leapfrog step taken by extra workgroups of the step launch
 // (swh_bflux.h): the caller asks for 'want' of them (0: none), the launcher places
 // ey = bf_rows() rows of its grid's width ahead of the tiles. part: the workgroups'
-// partial sums, room for 'cap' workgroups of 4 doubles; t_after: the end time of
+// partial sums, room for 'cap' workgroups of 12 doubles; t_after: the end time of
 // each step of the launch (NaN: from the device time).
 struct BfLines {
     int want = 0, cap = 0, ey = 0, n_ext = 2;
@@ -65,7 +65,7 @@ struct BfLines {
     DevScalars *sc = nullptr;
     double *part = nullptr;
     double dt = 0.0;
-    double t_after[2] = {0.0, 0.0};
+    double t_after[6] = {};
 };
 // Rows of line workgroups for a launch gx workgroups wide: enough for 'want' of them
 // (at least 4: one per side), within 'cap'; -1 if they do not fit.
@@ -152,6 +152,15 @@ struct LFArgs {
     double *g_val = nullptr;
     // single grid: the step's boundary-flux sums in extra workgroups of this launch
     BfLines bf;
+    // single grid, several steps per launch (launch_leapfrog_sg): bit n - 1 of mx_levels: step
+    // n updates max_stage; the pre-step UH/VH on the boundary-flux lines go to lb_out
+    // [step][side][lb_len], and the line workgroups (bf) sum those of the lb_levels steps in
+    // lb_in; the time of the gauge sample g_level, to be stored at g_time
+    int mx_levels = 0, lb_len = 0, lb_levels = 0;
+    T *lb_out = nullptr;
+    const T *lb_in = nullptr;
+    double *g_time = nullptr;
+    double g_t = 0.0;
 };
 
 // Kernel launchers (defined in the .hip files)
@@ -169,6 +178,18 @@ hipError_t launch_leapfrog2(const LFArgs<T> &a, int coriolis, int friction_mode,
 template <typename T, bool KAHAN>
 hipError_t launch_leapfrogn(const LFArgs<T> &a, int coriolis, int friction_mode, int truely_linear,
                             int linear_friction, int nsrc, int block_x, hipStream_t s, int prefetch, int ns);
+
+// ns (3 or 5; FP64: 3) fused steps of a single grid per launch, with max_stage, boundary
+// fluxes and (truely-linear 'linear': a.g_n) one gauge sample inside; the boundary-flux sums
+// of the launch's steps are taken by the next launch, or by launch_bf_flush after the last.
+template <typename T, bool KAHAN>
+hipError_t launch_leapfrog_sg(const LFArgs<T> &a, int coriolis, int friction_mode, int truely_linear,
+                              int linear_friction, int ns, hipStream_t s);
+template <typename T>
+hipError_t launch_bf_flush(const BfLines &b, int nx, int ny, const T *lines, int len_max, int levels, hipStream_t s);
+// Rows per strip of a fused launch of ns steps over n grids of nx * ny: the least time by
+// rows walked and rounds of resident wavefronts, at most 'most' rows.
+int fused_rows(int nx, int ny, int n, int ns, int own, int most);
 
 // Plain streaming copy of 'bytes' (a multiple of 16) for measurement.
 hipError_t launch_probe_copy(const void *src, void *dst, long long bytes, hipStream_t s);

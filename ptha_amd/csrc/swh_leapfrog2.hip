@@ -12,218 +12,15 @@
 // UH from memory); each lane owns one column and marches up a strip of rows. At
 // row m it forms step 1 at row m (stage, UH) and m-1 (VH), then step 2 at row m-1
 // (stage, UH) and m-2 (VH), and writes row m-2. East/west neighbours come
-// from the adjacent lanes (cross-lane permutes, no LDS tile, no barriers); the
+// from the adjacent lanes (lane moves, no LDS tile, no barriers); the
 // stencil reaches one column each way per step, which the 3 halo lanes cover.
 // Rows below/above the strip are recomputed by the strip itself (3 extra rows).
 #include <atomic>
 
-#include "swh_bflux.h"
+#include "swh_lf_fused.h"
 #include "swh_launch.h"
 
 namespace swh {
-
-namespace {
-
-constexpr int kOwn = 61;   // columns a wavefront writes (lanes 1..61)
-
-// Lane shifts across the wavefront (the lane at the open end keeps its own value).
-// Call them on every lane, outside lane-dependent conditions: a lane that does not
-// execute the shuffle leaves the lane reading from it with an undefined value.
-template <typename T>
-__device__ __forceinline__ T shl1(T v) { return __shfl_down(v, 1); }   // value of lane + 1
-template <typename T>
-__device__ __forceinline__ T shr1(T v) { return __shfl_up(v, 1); }     // value of lane - 1
-
-// Per-row coefficients (uniform across the wavefront), loaded at a clamped row so
-// the loads are always in bounds; 'interior' / 'valid' say whether the row updates.
-template <typename T>
-struct RowCo {
-    T sa, cu, cv, fu, fv, dbe_lo, dbe_hi;   // dbe_lo = dbe(j), dbe_hi = dbe(j+1)
-    bool interior, valid;                   // stage row (1..ny-2), momentum row (0..ny-2)
-};
-
-// A value that is the same on every lane (a row coefficient), kept in scalar registers.
-__device__ __forceinline__ float uniform(float v)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-__device__ __forceinline__ double uniform(double v)
-{
-    const long long b = __builtin_bit_cast(long long, v);
-    const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffff));
-    const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-
-template <typename T>
-__device__ __forceinline__ RowCo<T> row_co(const LFArgs<T> &a, int r)
-{
-    const int rc = min(max(r, 0), a.ny - 1);
-    RowCo<T> q;
-    q.sa = a.rc.sa[rc];
-    q.cu = a.rc.cu[rc];
-    q.cv = a.rc.cv[rc];
-    q.fu = a.rc.fu[rc];
-    q.fv = a.rc.fv[rc];
-    q.dbe_lo = a.rc.dbe[rc];
-    q.dbe_hi = a.rc.dbe[rc + 1];
-    q.interior = r > 0 && r < a.ny - 1;
-    q.valid = r >= 0 && r < a.ny - 1;
-    return q;
-}
-
-// row_co for a row that is the same on every lane of the wavefront (the fused n-step
-// kernel's rows), FP64: the coefficients in scalar registers, so that the rows carried
-// across iterations take no vector registers (150 -> 105 VGPRs at three steps, a fourth
-// wavefront per SIMD, FP64 batch +3 %). FP32 keeps them as the compiler places them: its
-// loop is issue-bound and the scalar-register spills this adds cost more than the
-// wavefront it gains (-7 %). Not for per-lane rows (step1_cell).
-template <typename T>
-__device__ __forceinline__ RowCo<T> row_co_u(const LFArgs<T> &a, int r)
-{
-    RowCo<T> q = row_co(a, r);
-    if (sizeof(T) == 4) return q;
-    q.sa = uniform(q.sa);
-    q.cu = uniform(q.cu);
-    q.cv = uniform(q.cv);
-    q.fu = uniform(q.fu);
-    q.fv = uniform(q.fv);
-    q.dbe_lo = uniform(q.dbe_lo);
-    q.dbe_hi = uniform(q.dbe_hi);
-    return q;
-}
-
-// New stage (include.f90:97-113), computed on every lane and kept where the cell
-// is interior; no stage boundary in this kernel.
-template <typename T, bool KAHAN>
-__device__ __forceinline__ void stage_cell(bool interior, T sa, T dle_i, T dbe_lo, T dbe_hi, T s, T c, T uh, T uhm,
-                                           T vh, T vhm, T &sn, T &cn)
-{
-    const T delta = sa * ((uh - uhm) * dle_i + (vh * dbe_hi - vhm * dbe_lo));
-    T t, cc;
-    if (KAHAN) {
-        const T y = -delta - c;
-        t = s + y;
-        cc = (t - s) - y;
-    } else {
-        t = s - delta;
-        cc = T(0);
-    }
-    sn = interior ? t : s;
-    cn = interior ? cc : c;
-}
-
-// Depth at a face of the truely-linear scheme (include.f90:265-280) from the elevations
-// of its two cells (e_far: the east or north one); it depends on the elevation alone.
-template <typename T>
-__device__ __forceinline__ T tl_face_depth(T e_near, T e_far, T msl)
-{
-    const T MIN = T(kMinDepth), HALF = T(0.5);
-    return (e_near < -MIN + msl && e_far < -MIN + msl) ? msl - HALF * (e_far + e_near) : T(0);
-}
-
-// UH at (ii + 1/2, j) from the new stage of cells ii, ii+1 and the pre-step VH of
-// rows j-1 (vhm0, vhm1 at ii, ii+1) and j (vh0, vh1). HPRE (truely linear only): e0
-// carries the face depth h_iph itself (tl_face_depth of the two elevations), e1 unused.
-template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool HPRE = false>
-__device__ __forceinline__ T mom_u(const LFArgs<T> &a, bool valid, T cu, T fu, T dle_ip1, T fwu, T uh_old, T s0,
-                                   T c0, T s1, T c1, T e0, T e1, T vhm0, T vhm1, T vh0, T vh1)
-{
-    static_assert(TL || !HPRE, "precomputed face depths are for the truely-linear scheme");
-    const T MIN = T(kMinDepth), HALF = T(0.5), msl = a.msl;
-    T h_iph, wet_iph;
-    if (TL) {
-        h_iph = HPRE ? e0 : tl_face_depth(e0, e1, msl);
-        wet_iph = T(1);
-    } else {
-        h_iph = (s0 - e0 > MIN && s1 - e1 > MIN) ? HALF * ((s1 + s0) - (e1 + e0)) : T(0);
-        wet_iph = h_iph > T(0) ? T(1) : T(0);
-    }
-    T ds_i = s1 - s0;
-    if (KAHAN) ds_i = ds_i - (c1 - c0);
-    T uh_new = uh_old * wet_iph - cu * h_iph * ds_i * dle_ip1;
-    if (COR || FRIC) {
-        const T vh_jmh = HALF * (vhm0 + vhm1);
-        const T vh_jph = HALF * (vh0 + vh1);
-        if (COR) {
-            const T dhc = fu * (h_iph > T(0) ? T(1) : T(0));
-            uh_new = uh_new + dhc * (vh_jmh + vh_jph);
-        }
-        if (FRIC) {
-            const T vbar = HALF * (vh_jmh + vh_jph);
-            const T fmu = T(1) / (T(1) + a.dt_lfc + a.dt * fwu * (sqrt(uh_old * uh_old + vbar * vbar)));
-            uh_new = fmu * uh_new;
-        }
-    }
-    if (LINF) uh_new = a.lin_fric_mult * uh_new;
-    return valid ? uh_new : uh_old;
-}
-
-// VH at (ii, j + 1/2) from the new stage of rows j, j+1 and the pre-step UH of
-// row j (uh_i at ii, uh_im1 at ii-1) and row j+1 (uhu_i, uhu_im1). HPRE: e0 carries
-// h_jph itself, eu unused.
-template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool HPRE = false>
-__device__ __forceinline__ T mom_v(const LFArgs<T> &a, bool valid, T cv, T fv, T dbe_hi, T fwv, T vh_old, T s0, T c0,
-                                   T sup, T cup, T e0, T eu, T uh_i, T uh_im1, T uhu_i, T uhu_im1)
-{
-    static_assert(TL || !HPRE, "precomputed face depths are for the truely-linear scheme");
-    const T MIN = T(kMinDepth), HALF = T(0.5), msl = a.msl;
-    T h_jph, wet_jph;
-    if (TL) {
-        h_jph = HPRE ? e0 : tl_face_depth(e0, eu, msl);
-        wet_jph = T(1);
-    } else {
-        h_jph = (sup - eu > MIN && s0 - e0 > MIN) ? HALF * ((sup + s0) - (eu + e0)) : T(0);
-        wet_jph = h_jph > T(0) ? T(1) : T(0);
-    }
-    T ds_j = sup - s0;
-    if (KAHAN) ds_j = ds_j - (cup - c0);
-    T vh_new = vh_old * wet_jph - cv * h_jph * ds_j * dbe_hi;
-    if (COR || FRIC) {
-        const T uh_ij = HALF * (uh_i + uh_im1);
-        const T uh_ijp1 = HALF * (uhu_i + uhu_im1);
-        if (COR) {
-            const T dhcj = fv * (h_jph > T(0) ? T(1) : T(0));
-            vh_new = vh_new - dhcj * (uh_ij + uh_ijp1);
-        }
-        if (FRIC) {
-            const T ubar = HALF * (uh_ij + uh_ijp1);
-            const T fmv = T(1) / (T(1) + a.dt_lfc + a.dt * fwv * (sqrt(vh_old * vh_old + ubar * ubar)));
-            vh_new = fmv * vh_new;
-        }
-    }
-    if (LINF) vh_new = a.lin_fric_mult * vh_new;
-    return valid ? vh_new : vh_old;
-}
-
-}  // namespace
-
-// The tile (column block, strip, source) of this workgroup. Workgroups are dispatched
-// to the 8 XCDs (each with its own L2) round-robin by linear index; in XCD order the
-// i-th workgroup on an XCD takes the i-th tile of that XCD's contiguous range of tiles,
-// ordered columns fastest, then the sources of a group of 'group' sources, then
-// strips, then groups. Neighbouring tiles of a strip, the sources of a group (which
-// read the same elevation and row coefficients) and the next strip (which reads the
-// halo rows of this one) thus run on the same L2 shortly after one another.
-// ey: rows of workgroups ahead of the tiles that do other work (single grid only).
-__device__ __forceinline__ void lf2_tile(int order, int group, int ey, int &bx, int &by, int &bz)
-{
-    bx = blockIdx.x; by = (int)blockIdx.y - ey; bz = blockIdx.z;
-    if (!order) return;
-    const unsigned gx = gridDim.x, gy = gridDim.y - ey, gz = gridDim.z;
-    const unsigned B = gx * gy * gz;
-    const unsigned b = blockIdx.x + gx * ((blockIdx.y - ey) + gy * blockIdx.z);
-    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
-    const unsigned L = xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
-    const unsigned G = (unsigned)group;
-    const unsigned gi = L / (gx * gy * G);                 // source group
-    const unsigned within = L - gi * (gx * gy * G);
-    const unsigned Gi = min(G, gz - gi * G);               // sources in this group (the last may be short)
-    const unsigned t = within / gx;
-    bx = (int)(within - t * gx);
-    bz = (int)(gi * G + t % Gi);
-    by = (int)(t / Gi);
-}
 
 template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF>
 __device__ __forceinline__ void step1_cell(const LFArgs<T> &a, const T *__restrict__ S, const T *__restrict__ C,
@@ -381,227 +178,6 @@ __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
         e_pp = e_p; e_p = e; e_p_r = e_r;
         q_pp = q_p; q_p = q;
         fw_u_p = fw_u1; fw_v_p = fw_v1;
-    }
-}
-
-// NS fused steps per launch (NS = 3: the state is read and written once per three
-// steps). The same per-cell operations as the one-step kernel, scheduled as in
-// leapfrog2_kernel but for any number of levels: at row m, level n (the state after n
-// steps) forms its stage and UH at row m-n+1 and its VH at row m-n from level n-1,
-// whose stage and UH of row m-n+1 were formed in the previous iteration (level 0: the
-// row loaded now) and whose VH of rows m-n+1 (this iteration) and m-n (the previous
-// one) are at hand; row m-NS of level NS is written. Each level consumes one lane
-// of the wavefront to the west (UH(i-1)) and one to the east (stage(i+1), VH(i+1)), so a
-// wavefront owns 65 - 2 NS of its 64 columns; each strip recomputes NS rows below and
-// NS - 1 above it.
-template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool PF, int NS, bool GS = false>
-__global__ __launch_bounds__(256, (GS && sizeof(T) == 4) ? 4 : 1) void leapfrogn_kernel(LFArgs<T> a)
-{
-    constexpr int OWN = 65 - 2 * NS;
-    int bx, by, bz;
-    lf2_tile(a.lf2_order, a.lf2_group, 0, bx, by, bz);
-    const int lane = threadIdx.x & 63;
-    const int wg = bx * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (wg * OWN >= a.nx) return;                        // whole wavefront past the east edge
-    const int col = wg * OWN - (NS - 1) + lane;          // column of this lane (may be < 0 or >= nx)
-    const int ci = min(max(col, 0), a.nx - 1);           // column it loads (clamped into the row)
-    const bool own = lane >= NS - 1 && lane < NS - 1 + OWN && col < a.nx;
-    const int j0 = by * a.rows_per_block;
-    if (j0 >= a.ny) return;
-    const int j1 = min(j0 + a.rows_per_block, a.ny);
-    const long long so = (long long)(bz + a.src_base) * a.src_stride;
-    const T *__restrict__ S = a.S + so;
-    const T *__restrict__ C = KAHAN ? a.C + so : nullptr;
-    const T *__restrict__ UH = a.UH + so;
-    const T *__restrict__ VH = a.VH + so;
-    T *__restrict__ So = a.So + so;
-    T *__restrict__ Co = KAHAN ? a.Co + so : nullptr;
-    T *__restrict__ UHo = a.UHo + so;
-    T *__restrict__ VHo = a.VHo + so;
-    const bool west = col == 0;                          // UH(i-1) clamps to UH(0) (include.f90:319-322)
-    const T dle_i = a.rc.dle[min(max(col, 0), a.nx)];
-    const T dle_ip1 = a.rc.dle[min(max(col + 1, 0), a.nx)];
-    const bool col_int = col > 0 && col < a.nx - 1;      // stage: interior column
-    const bool col_mom = col >= 0 && col < a.nx - 1;     // momentum: UH/VH of this column update
-    const int cf = min(max(col, 0), a.nx - 1);           // friction-work column
-    // the gauges in this lane's own column and rows j0..j1-1 (the host sees that there are
-    // at most two): indices + 1 in bytes 0 and 1 of gk (0: none), rows in the halves of gr
-    int gk = 0, gr = 0;
-    if (GS && own) {
-        for (int g = 0; g < a.g_n; g++) {
-            const int gi = a.g_ij[2 * g], gj = a.g_ij[2 * g + 1];
-            if (gi == col && gj >= j0 && gj < j1) {
-                if (gk == 0) { gk = g + 1; gr = gj; }
-                else { gk |= (g + 1) << 8; gr |= gj << 16; }
-            }
-        }
-    }
-
-    // carried between rows, per level n (0 = the loaded state)
-    T s_p[NS + 1], c_p[NS + 1];          // stage of level n at its stage row of the previous iteration
-    T uh_p[NS + 1], uh_p_l[NS + 1];      // UH of level n, previous iteration (level 0: row m-1), and its west value
-    T uh_pp[NS + 1], uh_pp_l[NS + 1];    // the iteration before that (levels >= 1)
-    T vh_p[NS + 1], vh_p_r[NS + 1];      // VH of level n, previous iteration, and its east value
-    T e_r[NS + 1], e_rr[NS + 1];         // elevation of row m-k and its east value
-    // truely linear: the face depths instead (they depend on the elevation alone, so each
-    // is formed once, when its row is loaded, not once per level): h_iph of row m-k,
-    // h_jph of the face above row m-1-k, and the elevation of row m-1
-    T hi_r[NS], hj_r[NS], e_prev = T(0);
-    T fwu_r[NS], fwv_r[NS];              // friction work: UH at row m-k, VH at row m-1-k
-    RowCo<T> q_r[NS + 1];                // row coefficients of row m-k
-#pragma unroll
-    for (int n = 0; n <= NS; n++) {
-        s_p[n] = T(0); c_p[n] = T(0); uh_p[n] = T(0); uh_p_l[n] = T(0); uh_pp[n] = T(0); uh_pp_l[n] = T(0);
-        vh_p[n] = T(0); vh_p_r[n] = T(0); e_r[n] = T(0); e_rr[n] = T(0);
-    }
-#pragma unroll
-    for (int n = 0; n < NS; n++) { hi_r[n] = T(0); hj_r[n] = T(0); }
-#pragma unroll
-    for (int n = 0; n < NS; n++) { fwu_r[n] = T(0); fwv_r[n] = T(0); }
-    const int m0 = j0 - NS + 1;
-    // the rings as they stand after row m0-1 (each iteration first slides them by one)
-#pragma unroll
-    for (int k = 0; k <= NS; k++) q_r[k] = row_co_u(a, m0 - 1 - k);
-    {
-        // the row below the first one: pre-step VH/UH/E of row m0-1
-        const int r = min(max(m0 - 1, 0), a.ny - 1);
-        const int o = r * a.pitch + ci;
-        vh_p[0] = VH[o];
-        uh_p[0] = UH[o];
-        e_r[0] = a.E[o];
-        vh_p_r[0] = shl1(vh_p[0]);
-        const T uh_sh = shr1(uh_p[0]);
-        uh_p_l[0] = west ? uh_p[0] : uh_sh;
-        e_rr[0] = shl1(e_r[0]);
-        e_prev = e_r[0];
-    }
-    auto load_row = [&](int m, T &s0, T &c0, T &uh0, T &vh0, T &e, T &uhw) {
-        const int mr = min(max(m, 0), a.ny - 1);
-        const int o = mr * a.pitch + ci;
-        s0 = S[o];
-        c0 = KAHAN ? C[o] : T(0);
-        uh0 = UH[o];
-        vh0 = VH[o];
-        e = a.E[o];
-        uhw = (lane == 0 && col > 0) ? UH[o - 1] : uh0;
-    };
-    T n_s0, n_c0, n_uh0, n_vh0, n_e, n_uhw;
-    if (PF) load_row(m0, n_s0, n_c0, n_uh0, n_vh0, n_e, n_uhw);
-    T cap_s = T(0), cap_c = T(0), cap_uh = T(0), cap_vh = T(0);   // the sampled level (gauges)
-
-    for (int m = m0; m <= j1 + NS - 1; m++) {
-        T s0, c0, uh0, vh0, e0, uh0_mem;
-        if (PF) {
-            s0 = n_s0; c0 = n_c0; uh0 = n_uh0; vh0 = n_vh0; e0 = n_e; uh0_mem = n_uhw;
-            if (m + 1 <= j1 + NS - 1) load_row(m + 1, n_s0, n_c0, n_uh0, n_vh0, n_e, n_uhw);
-        } else {
-            load_row(m, s0, c0, uh0, vh0, e0, uh0_mem);
-        }
-        // slide the rings of rows: index k now holds row m-k
-#pragma unroll
-        for (int k = NS; k >= 1; k--) q_r[k] = q_r[k - 1];
-        q_r[0] = row_co_u(a, m);
-        if constexpr (TL) {
-#pragma unroll
-            for (int k = NS - 1; k >= 1; k--) { hi_r[k] = hi_r[k - 1]; hj_r[k] = hj_r[k - 1]; }
-            hi_r[0] = tl_face_depth(e0, shl1(e0), a.msl);
-            hj_r[0] = tl_face_depth(e_prev, e0, a.msl);
-            e_prev = e0;
-        } else {
-#pragma unroll
-            for (int k = NS; k >= 1; k--) { e_r[k] = e_r[k - 1]; e_rr[k] = e_rr[k - 1]; }
-            e_r[0] = e0;
-            e_rr[0] = shl1(e0);
-        }
-        if (FRIC) {
-#pragma unroll
-            for (int k = NS - 1; k >= 1; k--) { fwu_r[k] = fwu_r[k - 1]; fwv_r[k] = fwv_r[k - 1]; }
-            const int mr = min(max(m, 0), a.ny - 1);
-            fwu_r[0] = a.fwU[mr * a.pitch + cf];
-            fwv_r[0] = a.fwV[min(max(m - 1, 0), a.ny - 1) * a.pitch + cf];
-        }
-        // level 0 at row m (the loaded row); UH(i-1) from the west lane, lane 0 from memory
-        const T uh0_sh = shr1(uh0);
-        const T uh0_l = west ? uh0 : (lane == 0 ? uh0_mem : uh0_sh);
-        // inputs of the level being formed: stage/UH of the level below at this level's
-        // stage row, its VH there (cur) and one row below (below)
-        T in_s = s0, in_c = c0, in_uh = uh0, in_uh_l = uh0_l;
-        T in_uhb = uh_p[0], in_uhb_l = uh_p_l[0];     // UH of the level below one row lower
-        T vh_cur = vh0, vh_cur_r = shl1(vh0);
-        T out_s = T(0), out_c = T(0), out_uh = T(0), out_vh = T(0);
-#pragma unroll
-        for (int n = 1; n <= NS; n++) {
-            const int r = m - n + 1;                  // this level's stage/UH row
-            const RowCo<T> &q = q_r[n - 1];           // row r
-            const RowCo<T> &qb = q_r[n];              // row r-1
-            // VH of the level below at row r-1, clamped to row r at the southern edge
-            const T vhb = r > 0 ? vh_p[n - 1] : vh_cur, vhb_r = r > 0 ? vh_p_r[n - 1] : vh_cur_r;
-            T sn, cn;
-            stage_cell<T, KAHAN>(col_int && q.interior, q.sa, dle_i, q.dbe_lo, q.dbe_hi, in_s, in_c, in_uh, in_uh_l,
-                                 vh_cur, vhb, sn, cn);
-            const T sn_r = shl1(sn);
-            const T cn_r = KAHAN ? shl1(cn) : T(0);
-            // the face depths of this level's rows (truely linear: precomputed), or the
-            // elevations they are formed from
-            const T fu_a = TL ? hi_r[n - 1] : e_r[n - 1], fu_b = TL ? T(0) : e_rr[n - 1];
-            const T fv_a = TL ? hj_r[n - 1] : e_r[n], fv_b = TL ? T(0) : e_r[n - 1];
-            const T uhn = mom_u<T, KAHAN, COR, FRIC, TL, LINF, TL>(a, col_mom && q.valid, q.cu, q.fu, dle_ip1,
-                                                                    FRIC ? fwu_r[n - 1] : T(0), in_uh, sn, cn, sn_r,
-                                                                    cn_r, fu_a, fu_b, vhb, vhb_r, vh_cur, vh_cur_r);
-            // VH at row r-1: stage of this level at rows r-1 (previous iteration) and r,
-            // UH of the level below at rows r-1 and r
-            const T vhn = mom_v<T, KAHAN, COR, FRIC, TL, LINF, TL>(a, col_mom && qb.valid, qb.cv, qb.fv, qb.dbe_hi,
-                                                                    FRIC ? fwv_r[n - 1] : T(0), vh_p[n - 1], s_p[n],
-                                                                    c_p[n], sn, cn, fv_a, fv_b, in_uhb, in_uhb_l,
-                                                                    in_uh, in_uh_l);
-            if (GS && n == a.g_level) {
-                // the sampled level's values at this iteration's rows
-                cap_s = sn; cap_c = cn; cap_uh = uhn; cap_vh = vhn;
-            }
-            const T uhn_sh = shr1(uhn);
-            const T uhn_l = west ? uhn : uhn_sh;
-            const T vhn_r = shl1(vhn);
-            // the level below's VH of this iteration becomes its 'previous' one
-            if (n == 1) {
-                // level 0: the loaded row's UH/VH become row m-1's
-                uh_p[0] = uh0; uh_p_l[0] = uh0_l;
-            }
-            vh_p[n - 1] = vh_cur; vh_p_r[n - 1] = vh_cur_r;
-            if (n == NS) {
-                out_s = s_p[n]; out_c = c_p[n]; out_uh = uh_p[n]; out_vh = vhn;
-            }
-            // inputs of level n+1: this level's stage/UH of the previous iteration (row
-            // m-n), this level's VH now (row m-n)
-            in_s = s_p[n]; in_c = c_p[n]; in_uh = uh_p[n]; in_uh_l = uh_p_l[n];
-            in_uhb = uh_pp[n]; in_uhb_l = uh_pp_l[n];
-            vh_cur = vhn; vh_cur_r = vhn_r;
-            // slide this level
-            s_p[n] = sn; c_p[n] = cn;
-            uh_pp[n] = uh_p[n]; uh_pp_l[n] = uh_p_l[n];
-            uh_p[n] = uhn; uh_p_l[n] = uhn_l;
-        }
-        vh_p[NS] = vh_cur; vh_p_r[NS] = vh_cur_r;
-        if (GS && gk) {
-            // the gauge samples after the launch's g_level-th step: stage and UH of row r,
-            // VH of row r-1
-            const int r = m - a.g_level + 1;
-            double *v = a.g_val + ((long long)(bz + a.src_base) * a.g_max + a.g_sample) * 3 * a.g_n;
-            const double st = KAHAN ? (double)cap_s - (double)cap_c : (double)cap_s;
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int g = ((gk >> (8 * q)) & 255) - 1, row = (gr >> (16 * q)) & 0xffff;
-                if (g >= 0 && r == row) { v[g] = st; v[a.g_n + g] = (double)cap_uh; }
-                if (g >= 0 && r - 1 == row) v[2 * a.g_n + g] = (double)cap_vh;
-            }
-        }
-        const int k = m - NS;
-        if (own && k >= j0 && k < j1) {
-            const int ow = k * a.pitch + col;
-            So[ow] = out_s;
-            if (KAHAN) Co[ow] = out_c;
-            UHo[ow] = out_uh;
-            VHo[ow] = out_vh;
-        }
     }
 }
 

@@ -1,5 +1,6 @@
 """GPU: batches with the strip height left to the launch (chosen from the sources still
-running), on grids from a few rows to more than a strip, with sources that stop at
+running), on grids from a few rows to more than a strip and to one
+that fills the device with its deeper launches, with sources that stop at
 different steps so that the height changes between launches: each source's final state and
 gauge series equal those of the same source stepped alone, one step per launch, bit for
 bit (both precisions)."""
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32k"])
 @pytest.mark.parametrize("nx,ny,steps", [(7, 5, (3, 9)), (56, 13, (23, 7, 1)), (130, 97, (40, 12, 0, 33, 21)),
-                                         (611, 300, (17, 6))])
+                                         (611, 300, (17, 6)), (1300, 1200, (14, 9, 14, 3))])
 def test_rows_chosen_per_launch(precision, nx, ny, steps):
     print("CASE batch rows", precision, nx, ny, steps, flush=True)
     rng = np.random.default_rng(nx + ny)
