@@ -2820,11 +2820,25 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
     const int TE = superpose_event_tile();
     const int Kpad = (b->nsrc + 3) / 4 * 4;
     const long long ncol = summary == SWH_SUPERPOSE_SERIES ? (long long)b->gmax * 3 * b->ng : b->ng;
+    // as lists of each event's sources (few of all of them), or a dense weight matrix
+    const bool lists = superpose_lists_fit(b->nsrc, n_events, event_ptr[n_events], event_w != nullptr);
     // events per launch: bounded device output (<= 2^28 doubles) and weight matrix
-    long long chunk = std::max<long long>(TE, ((1LL << 28) / std::max<long long>(ncol, Kpad)) / TE * TE);
+    const long long row = lists ? ncol : std::max<long long>(ncol, Kpad);
+    long long chunk = std::max<long long>(TE, ((1LL << 28) / row) / TE * TE);
     chunk = std::min<long long>(chunk, (n_events + TE - 1) / TE * TE);
     double *d_w = nullptr, *d_scale = nullptr, *d_out = nullptr, *d_m = nullptr;
     int *d_nv = nullptr, *d_flags = nullptr;
+    SupList *d_recs = nullptr;
+    unsigned short *d_lists = nullptr;
+    // list entries (quads of sources) of the largest launch, two spare ones at the end
+    long long quads_most = 0;
+    if (lists)
+        for (long long e0 = 0; e0 < n_events; e0 += chunk) {
+            long long n = 0;
+            for (long long e = e0; e < std::min<long long>(e0 + chunk, n_events); e++)
+                n += (event_ptr[e + 1] - event_ptr[e] + 3) / 4;
+            quads_most = std::max(quads_most, n + 2);
+        }
     // slots whose series hold a non-finite value (a source that blew up): only the
     // events that contain them may see it
     std::vector<int> flagged(b->nsrc, 0);
@@ -2839,8 +2853,14 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
         if (he != hipSuccess) rc = hip_fail(he, "superposition non-finite scan", __FILE__, __LINE__);
         for (int k = 0; k < b->nsrc; k++) any_flagged |= flagged[k] != 0;
     }
-    if (!rc) rc = dmalloc((void **)&d_w, sizeof(double) * chunk * Kpad);
-    if (!rc && any_flagged) rc = dmalloc((void **)&d_m, sizeof(double) * chunk * Kpad);
+    if (!rc && lists) {
+        if (event_w) rc = dmalloc((void **)&d_w, sizeof(double) * 4 * quads_most);
+        if (!rc) rc = dmalloc((void **)&d_lists, sizeof(unsigned short) * 4 * quads_most);
+        if (!rc) rc = dmalloc((void **)&d_recs, sizeof(SupList) * chunk);
+    } else if (!rc) {
+        rc = dmalloc((void **)&d_w, sizeof(double) * chunk * Kpad);
+        if (!rc && any_flagged) rc = dmalloc((void **)&d_m, sizeof(double) * chunk * Kpad);
+    }
     if (!rc) rc = dmalloc((void **)&d_scale, sizeof(double) * chunk);
     if (!rc) rc = dmalloc((void **)&d_nv, sizeof(int) * chunk);
     if (!rc) rc = dmalloc((void **)&d_out, sizeof(double) * chunk * ncol);
@@ -2849,11 +2869,15 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
     if (!rc && (hipEventCreate(&t0) != hipSuccess || hipEventCreate(&t1) != hipSuccess))
         rc = fail(SWH_EHIP, "hipEventCreate failed");
     std::vector<double> W, M, scale;
-    std::vector<int> nv;
+    std::vector<int> nv, order;
+    std::vector<SupList> recs;
+    std::vector<unsigned short> ls;
     for (long long e0 = 0; !rc && e0 < n_events; e0 += chunk) {
         const int E = (int)std::min<long long>(chunk, n_events - e0);
-        W.assign((size_t)chunk * Kpad, 0.0);
-        if (any_flagged) M.assign((size_t)chunk * Kpad, 0.0);
+        if (!lists) {
+            W.assign((size_t)chunk * Kpad, 0.0);
+            if (any_flagged) M.assign((size_t)chunk * Kpad, 0.0);
+        }
         scale.assign(chunk, 0.0);
         nv.assign(chunk, 0);
         int smax = 1;
@@ -2864,8 +2888,10 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
                 const int slot = b->slot_of[event_src[q]];
                 // uniform slip: unit weights, the slip scales the sum
                 // (sum_tsunami_unit_sources.R:658-669); stochastic: per-source slips (:672-687)
-                W[(size_t)e * Kpad + slot] += event_w ? event_w[q] : 1.0;
-                if (any_flagged && flagged[slot]) M[(size_t)e * Kpad + slot] = 1.0;
+                if (!lists) {
+                    W[(size_t)e * Kpad + slot] += event_w ? event_w[q] : 1.0;
+                    if (any_flagged && flagged[slot]) M[(size_t)e * Kpad + slot] = 1.0;
+                }
                 n_e = std::min(n_e, ns_slot[slot]);
             }
             scale[e] = event_slip ? event_slip[ev] : 1.0;
@@ -2873,10 +2899,41 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
             nvalid[ev] = n_e;
             smax = std::max(smax, n_e);
         }
-        if (hipMemcpy(d_w, W.data(), sizeof(double) * W.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        if (lists) {
+            // longest lists first, those of like length together (a counting sort by quads)
+            auto quads_of = [&](int e) { return (event_ptr[e0 + e + 1] - event_ptr[e0 + e] + 3) / 4; };
+            int longest = 0;
+            for (int e = 0; e < E; e++) longest = std::max(longest, quads_of(e));
+            std::vector<int> at(longest + 2, 0);
+            for (int e = 0; e < E; e++) at[longest - quads_of(e) + 1]++;
+            for (int q = 0; q <= longest; q++) at[q + 1] += at[q];
+            order.resize(E);
+            recs.resize(E);
+            for (int e = 0; e < E; e++) order[at[longest - quads_of(e)]++] = e;
+            ls.assign(4 * quads_most, (unsigned short)b->nsrc);
+            if (event_w) W.assign(4 * quads_most, 0.0);
+            int nq = 0;
+            for (int q = 0; q < E; q++) {
+                const int ev = (int)e0 + order[q];
+                recs[q] = SupList{order[q], nq, quads_of(order[q]), nv[order[q]], scale[order[q]]};
+                size_t o = (size_t)4 * nq;
+                for (int k = event_ptr[ev]; k < event_ptr[ev + 1]; k++, o++) {
+                    ls[o] = (unsigned short)b->slot_of[event_src[k]];
+                    if (event_w) W[o] = event_w[k];
+                }
+                nq += quads_of(order[q]);
+            }
+            if (hipMemcpy(d_lists, ls.data(), sizeof(unsigned short) * ls.size(), hipMemcpyHostToDevice) != hipSuccess ||
+                hipMemcpy(d_recs, recs.data(), sizeof(SupList) * E, hipMemcpyHostToDevice) != hipSuccess) {
+                rc = fail(SWH_EHIP, "superposition upload failed");
+                break;
+            }
+        }
+        if ((!W.empty() &&
+             hipMemcpy(d_w, W.data(), sizeof(double) * W.size(), hipMemcpyHostToDevice) != hipSuccess) ||
             hipMemcpy(d_scale, scale.data(), sizeof(double) * chunk, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy(d_nv, nv.data(), sizeof(int) * chunk, hipMemcpyHostToDevice) != hipSuccess ||
-            (any_flagged &&
+            (d_m &&
              hipMemcpy(d_m, M.data(), sizeof(double) * M.size(), hipMemcpyHostToDevice) != hipSuccess)) {
             rc = fail(SWH_EHIP, "superposition upload failed");
             break;
@@ -2887,9 +2944,15 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
         a.W = d_w; a.Kpad = Kpad; a.E = E; a.scale = d_scale; a.nvalid = d_nv; a.msl = msl;
         a.s_chunk = 16; a.s_max = std::min(smax, b->gmax);
         a.out = d_out;
-        a.M = any_flagged ? d_m : nullptr;
+        a.M = d_m;
+        if (lists) {
+            a.recs = d_recs; a.lists = d_lists; a.list_w = event_w ? d_w : nullptr;
+            a.flagged = any_flagged ? 1 : 0;
+        }
         hipError_t he = hipEventRecord(t0, g->stream);
-        if (he == hipSuccess) he = launch_superpose(a, summary == SWH_SUPERPOSE_SERIES ? 0 : 1, g->stream);
+        const int mode = summary == SWH_SUPERPOSE_SERIES ? 0 : 1;
+        if (he == hipSuccess)
+            he = lists ? launch_superpose_lists(a, mode, g->stream) : launch_superpose(a, mode, g->stream);
         if (he == hipSuccess) he = hipEventRecord(t1, g->stream);
         if (he == hipSuccess) he = hipEventSynchronize(t1);
         float ms = 0.0f;
@@ -2904,7 +2967,7 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
     }
     if (t0) (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);
-    dfree(d_w); dfree(d_scale); dfree(d_nv); dfree(d_out); dfree(d_m); dfree(d_flags);
+    dfree(d_w); dfree(d_scale); dfree(d_nv); dfree(d_out); dfree(d_m); dfree(d_flags); dfree(d_lists); dfree(d_recs);
     if (!rc && kernel_ms) *kernel_ms = total_ms;
     return rc;
 }

@@ -204,6 +204,11 @@ hipError_t launch_plane_to_dense(const T *src, const T *comp, double *dst, int n
 hipError_t launch_probe_math(const double *x, const double *y, const double *t, double *pw, double *sn, int n,
                              hipStream_t s);
 
+struct alignas(8) SupList {
+    int event, begin, n, nvalid;
+    double scale;
+};
+
 // Events from unit-source gauge series (swh_superpose.hip): out = W * (X - msl on the
 // stage) scaled and shifted per event.
 struct SupArgs {
@@ -222,6 +227,15 @@ struct SupArgs {
     // event has such a slot (non-finite values then enter the product as 0, and the
     // outputs that an event's non-finite members reach are NaN)
     const double *M = nullptr;
+    // events as lists (superpose_lists_fit; W, M, scale and nvalid are then not used): recs
+    // (E of them, lists of like length together) give an event's entries of four slots
+    // each, lists[4 begin..4 (begin + n)), their weights in list_w (null: 1); an unused place
+    // names slot nsrc (zeros); two spare entries end the lists. flagged: non-finite values
+    // enter as NaN
+    const SupList *recs = nullptr;
+    const unsigned short *lists = nullptr;
+    const double *list_w = nullptr;
+    int flagged = 0;
 };
 // Forcing patch on a finite-volume state after update_U (forcing_mod.f90:80-156):
 // the fraction of [start, end] that the stage (time - stage_dt, time] covers, read
@@ -321,6 +335,8 @@ hipError_t launch_add_scaled(T *E, const T *fE, int pitch, int i0, int i1, int j
 
 // rows of the event tile (W, scale and nvalid must hold a multiple of it)
 int superpose_event_tile();
+bool superpose_lists_fit(int nsrc, long long n_events, long long entries, bool weights);
+hipError_t launch_superpose_lists(const SupArgs &a, int mode, hipStream_t s);
 hipError_t launch_superpose(const SupArgs &a, int mode, hipStream_t s);
 // flags[slot] = 1 where the slot's series (slot_stride values each) holds a non-finite
 // value; flags must start at 0.
