@@ -43,17 +43,24 @@ __device__ __forceinline__ T face_depth(T e0, T e_far, T msl)
 
 // One transposed step, fused and column-marching. Each lane owns one column (a
 // wavefront owns 61: lane 0 is the western halo, lanes 62-63 the eastern one) and
-// marches up a strip of rows, keeping the last three rows in registers; east and west
+// marches up a strip of rows, keeping what two rows share in registers; east and west
 // neighbours come from the adjacent lanes. At row m (loaded now) it forms
 //   h_iph(m), aU mu_U(m) = cu h_iph dle(i+1) LF lU,      (and its west neighbour's)
 //   h_jph(m-1), aV mu_V(m-1) = cv h_jph dbe(j+1) LF lV,
+//   the Coriolis products bU mu_U(m), bV mu_V(m-1) and their west / east neighbours',
 //   pass 1 at row m-1: lS_in = lS + aU mu_U(i) - aU mu_U(i-1) + aV mu_V(j) - aV mu_V(j-1),
 //   pass 2 at row m-2: lU_in, lV_in = identity / Coriolis transpose of LF l' plus the
 //   divergence transpose of lS_in (its own, its east neighbour's, the row above's),
 // with the operations and their order of the two-pass form, on 0 <= i < nx-1,
-// 0 <= j < ny-1 for the momentum points and the interior for the stage. Each strip
-// recomputes one row below and two above it; the next two rows' loads are in flight
-// while a row is computed.
+// 0 <= j < ny-1 for the momentum points and the interior for the stage: a term of a point
+// outside is zeroed where it is formed. Each strip recomputes one row below and two above it.
+//
+// What bounds it: on grids of up to about 1024 x 1024 the chain of one strip's rows, so a row
+// is short: each product is formed once, by the lane and in the row that it belongs to (its
+// neighbour's is a lane move, the other row's is carried), 75 vector operations in FP32
+// (85 at the grid's edges) against 163 when every term was formed where it is used; and the
+// loads of the next two rows are issued before two rows are computed and looked at after
+// them. 1024 x 1024 FP32 13.0 -> 8.9 us a step, 300 x 300 6.1 -> 4.3.
 // Row coefficients of row r (loaded once per row at a clamped index, carried while the
 // row is in use): sa, cu, cv, fu, fv, dbe(r+1); mom: 0 <= r < ny-1 (momentum row),
 // in: 0 < r < ny-1 (stage row).
@@ -79,110 +86,107 @@ __device__ __forceinline__ AdjRow<T> adj_row(const AdjArgs<T> &a, int r)
     return q;
 }
 
-template <typename T, bool COR>
-__global__ __launch_bounds__(256) void adj_march_kernel(AdjArgs<T> a)
+template <typename T, bool COR, bool EDGE>
+__device__ __forceinline__ void adj_march(const AdjArgs<T> &a, int wg, int j0, int j1)
 {
-    const int lane = threadIdx.x & 63;
-    const int wg = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (wg * kAdjOwn >= a.nx) return;                    // whole wavefront past the east edge
-    const int col = wg * kAdjOwn - 1 + lane;             // may be -1 or >= nx
-    const int ci = min(max(col, 0), a.nx - 1);           // column it loads
-    const bool own = lane >= 1 && lane <= kAdjOwn && col < a.nx;
-    const int j0 = blockIdx.y * a.rows;
-    if (j0 >= a.ny) return;
-    const int j1 = min(j0 + a.rows, a.ny);
-    const int nx = a.nx, ny = a.ny;
-    const long long P = a.pitch;
+    const int lane = threadIdx.x & 63, nx = a.nx, ny = a.ny;
+    const int col = wg * kAdjOwn - 1 + lane;             // EDGE: may be -1 or >= nx
+    const int ci = EDGE ? min(max(col, 0), nx - 1) : col;
+    const bool own = lane >= 1 && lane <= kAdjOwn && (!EDGE || col < nx);
+    const bool cmom = !EDGE || (col >= 0 && col < nx - 1), cint = !EDGE || (col > 0 && col < nx - 1);
     const T LF = a.lin_fric_mult, HALF = T(0.5), msl = a.msl;
-    // column parts of the momentum-domain and interior predicates (i, i-1, i+1)
-    const bool cmom = col >= 0 && col < nx - 1, cmom_w = col - 1 >= 0 && col - 1 < nx - 1,
-               cmom_e = col + 1 >= 0 && col + 1 < nx - 1;
-    const bool cint = col > 0 && col < nx - 1, cint_e = col + 1 > 0 && col + 1 < nx - 1;
-    const T dle_i = a.rc.dle[min(max(col, 0), nx)], dle_ip1 = a.rc.dle[min(max(col + 1, 0), nx)];
-    const T mult_i = T(col == 0 ? 2 : 1);                // U(0,.) counted twice at i = 0
-
-    // carried rows (m-1, m-2, m-3 relative to the row loaded now)
-    T ls1 = T(0), lu1 = T(0), lv1 = T(0), e1 = T(0), hI1 = T(0), hIw1 = T(0), luw1 = T(0), aU1 = T(0), aUw1 = T(0);
-    T lu2 = T(0), lv2 = T(0), hI2 = T(0), hIw2 = T(0), luw2 = T(0), oS2 = T(0), lve2 = T(0), hJ2 = T(0),
-      hJe2 = T(0), aV2 = T(0);
-    T lv3 = T(0), lve3 = T(0), hJ3 = T(0), hJe3 = T(0);
-    AdjRow<T> q1 = adj_row(a, j0 - 2), q2 = adj_row(a, j0 - 3), q3 = adj_row(a, j0 - 4), n_q = adj_row(a, j0 - 1);
-
-    // the next two rows' loads are issued before this row is computed (two rows in flight)
-    auto load_row = [&](int m, T &ls, T &lu, T &lv, T &e) {
-        const long long o = (long long)min(max(m, 0), ny - 1) * P + ci;
-        ls = a.lS[o];
-        lu = a.lU[o];
-        lv = a.lV[o];
-        e = a.E[o];
+    const T dle_i = a.rc.dle[EDGE ? min(max(col, 0), nx) : col];
+    const T dle_ip1 = a.rc.dle[EDGE ? min(max(col + 1, 0), nx) : col + 1];
+    const T mult_i = T(EDGE && col == 0 ? 2 : 1);        // U(0,.) counted twice at i = 0
+    struct Row {
+        T ls, lu, lv, e;
     };
-    T n_ls, n_lu, n_lv, n_e, nn_ls, nn_lu, nn_lv, nn_e;
-    load_row(j0 - 1, n_ls, n_lu, n_lv, n_e);
-    load_row(j0, nn_ls, nn_lu, nn_lv, nn_e);
-    for (int m = j0 - 1; m <= j1 + 1; m++) {
-        const T ls0 = n_ls, lu0 = n_lu, lv0 = n_lv, e0 = n_e;
-        n_ls = nn_ls; n_lu = nn_lu; n_lv = nn_lv; n_e = nn_e;
-        if (m + 2 <= j1 + 1) load_row(m + 2, nn_ls, nn_lu, nn_lv, nn_e);
-        const AdjRow<T> q0 = n_q;
-        n_q = adj_row(a, m + 1);
-        const T e0e = shl1(e0);
-        // row m: h_iph and aU mu_U (own and the west neighbour's)
-        const T hI0 = face_depth(e0, e0e, msl);
-        const T hIw0 = shr1(hI0);
-        const T luw0 = shr1(lu0);
-        const T aU0 = (cmom && q0.mom) ? q0.cu * hI0 * dle_ip1 * (LF * lu0) : T(0);
+    auto load_row = [&](int m) {
+        const int o = min(EDGE ? max(m, 0) : m, ny - 1) * a.pitch + ci;
+        return Row{a.lS[o], a.lU[o], a.lV[o], a.E[o]};
+    };
+    // of rows m-1, m-2 (m-3): the loaded values, LF l', the pressure terms, the new stage
+    // adjoint (as written, and where it is an interior cell's), the Coriolis products
+    T ls1 = T(0), lu1 = T(0), lv1 = T(0), e1 = T(0), aU1 = T(0), aUw1 = T(0), mu1 = T(0), pu1 = T(0), puw1 = T(0);
+    T aV2 = T(0), oS2 = T(0), in2 = T(0), lu2 = T(0), lv2 = T(0), mu2 = T(0), mv2 = T(0), pu2 = T(0), puw2 = T(0),
+      pv2 = T(0), pve2 = T(0), pv3 = T(0), pve3 = T(0);
+    AdjRow<T> q1 = adj_row(a, j0 - 2), q2 = q1;
+    auto row = [&](const int m, const Row &in, const AdjRow<T> &q0) {
+        const T ls0 = in.ls, lu0 = in.lu, lv0 = in.lv, e0 = in.e;
+        // row m
+        const T hI0 = face_depth(e0, shl1(e0), msl);
+        const T mu0 = LF * lu0;
+        T aU0 = q0.cu * hI0 * dle_ip1 * mu0;
+        if (EDGE) aU0 = (cmom && q0.mom) ? aU0 : T(0);
         const T aUw0 = shr1(aU0);
-        // row m-1: h_jph and aV mu_V
+        // row m-1
         const T hJ1 = face_depth(e1, e0, msl);
-        const T hJe1 = shl1(hJ1);
-        const T lve1 = shl1(lv1);
-        const T aV1 = (cmom && q1.mom) ? q1.cv * hJ1 * q1.dbe1 * (LF * lv1) : T(0);
-        // pass 1 at row m-1 (aU mu_U(i-1) is zero outside the momentum domain: the west
-        // lane's value carries its own column's predicate)
+        const T mv1 = LF * lv1;
+        T aV1 = q1.cv * hJ1 * q1.dbe1 * mv1;
+        if (EDGE) aV1 = (cmom && q1.mom) ? aV1 : T(0);
         const T oS1 = (((ls1 + aU1) - aUw1) + aV1) - aV2;
-        const T oSe2 = shl1(oS2);
-        // pass 2 at row r = m-2
-        const int r = m - 2;
-        const bool mom = cmom && q2.mom;
-        T lu_o = mom ? LF * lu2 : lu2;
-        T lv_o = mom ? LF * lv2 : lv2;
-        if (cint && q2.in) {
-            lu_o -= q2.sa * dle_i * oS2;
-            lv_o -= q2.sa * q2.dbe1 * oS2;
-        }
-        if (cint_e && q2.in) lu_o += q2.sa * dle_ip1 * oSe2;
-        if (cint && q1.in) lv_o += q1.sa * q2.dbe1 * oS1;
+        const T in1 = !EDGE || (cint && q1.in) ? oS1 : T(0);
+        T pu0 = T(0), puw0 = T(0), pv1 = T(0), pve1 = T(0);
         if (COR) {
-            // UH(i,j) in VH'(k,l), l in {j, j-1}, k in {i, i+1} (U(0,.) twice at i = 0);
-            // row j-1 is no momentum row when j = 0
-            T acc = T(0);
-            if (cmom && q2.mom) acc += mult_i * (HALF * q2.fv * (hJ2 > T(0) ? T(1) : T(0))) * (LF * lv2);
-            if (cmom_e && q2.mom) acc += T(1) * (HALF * q2.fv * (hJe2 > T(0) ? T(1) : T(0))) * (LF * lve2);
-            if (cmom && q3.mom) acc += mult_i * (HALF * q3.fv * (hJ3 > T(0) ? T(1) : T(0))) * (LF * lv3);
-            if (cmom_e && q3.mom) acc += T(1) * (HALF * q3.fv * (hJe3 > T(0) ? T(1) : T(0))) * (LF * lve3);
-            lu_o -= acc;
-            // VH(i,j) in UH'(k,l), l in {j, j+1}, k in {i, i-1} (V(.,0) twice at j = 0)
-            acc = T(0);
-            const T mult_j = T(r == 0 ? 2 : 1);
-            if (cmom && q2.mom) acc += mult_j * (HALF * q2.fu * (hI2 > T(0) ? T(1) : T(0))) * (LF * lu2);
-            if (cmom_w && q2.mom) acc += mult_j * (HALF * q2.fu * (hIw2 > T(0) ? T(1) : T(0))) * (LF * luw2);
-            if (cmom && q1.mom) acc += T(1) * (HALF * q1.fu * (hI1 > T(0) ? T(1) : T(0))) * (LF * lu1);
-            if (cmom_w && q1.mom) acc += T(1) * (HALF * q1.fu * (hIw1 > T(0) ? T(1) : T(0))) * (LF * luw1);
-            lv_o += acc;
+            pu0 = (hI0 > T(0) ? HALF * q0.fu : T(0)) * mu0;
+            if (EDGE) pu0 = (cmom && q0.mom) ? pu0 : T(0);
+            puw0 = shr1(pu0);
+            pv1 = (hJ1 > T(0) ? HALF * q1.fv : T(0)) * mv1;
+            if (EDGE) pv1 = (cmom && q1.mom) ? pv1 : T(0);
+            pve1 = shl1(pv1);
+            if (EDGE) pv1 = mult_i * pv1;
+        }
+        // row m-2
+        const int r = m - 2;
+        const bool mom2 = !EDGE || (cmom && q2.mom);
+        T lu_o = (mom2 ? mu2 : lu2) - q2.sa * dle_i * in2;
+        T lv_o = (mom2 ? mv2 : lv2) - q2.sa * q2.dbe1 * in2;
+        lu_o += q2.sa * dle_ip1 * shl1(in2);
+        lv_o += q1.sa * q2.dbe1 * in1;
+        if (COR) {
+            const T mult_j = T(EDGE && r == 0 ? 2 : 1);  // V(.,0) counted twice at j = 0
+            lu_o -= (((T(0) + pv2) + pve2) + pv3) + pve3;
+            lv_o += (((T(0) + mult_j * pu2) + mult_j * puw2) + pu1) + puw1;
         }
         if (own && r >= j0 && r < j1) {
-            const long long ow = (long long)r * P + col;
+            const int ow = r * a.pitch + col;
             a.oS[ow] = oS2;
             a.oU[ow] = lu_o;
             a.oV[ow] = lv_o;
         }
-        // slide up one row
-        lv3 = lv2; lve3 = lve2; hJ3 = hJ2; hJe3 = hJe2;
-        lu2 = lu1; lv2 = lv1; hI2 = hI1; hIw2 = hIw1; luw2 = luw1; oS2 = oS1; lve2 = lve1; hJ2 = hJ1; hJe2 = hJe1;
-        aV2 = aV1;
-        ls1 = ls0; lu1 = lu0; lv1 = lv0; e1 = e0; hI1 = hI0; hIw1 = hIw0; luw1 = luw0; aU1 = aU0; aUw1 = aUw0;
-        q3 = q2; q2 = q1; q1 = q0;
+        pv3 = pv2; pve3 = pve2;
+        aV2 = aV1; oS2 = oS1; in2 = in1; lu2 = lu1; lv2 = lv1; mu2 = mu1; mv2 = mv1;
+        pu2 = pu1; puw2 = puw1; pv2 = pv1; pve2 = pve1;
+        ls1 = ls0; lu1 = lu0; lv1 = lv0; e1 = e0; aU1 = aU0; aUw1 = aUw0; mu1 = mu0; pu1 = pu0; puw1 = puw0;
+        q2 = q1; q1 = q0;
+    };
+    Row ra = load_row(j0 - 1), rb = load_row(j0);
+    AdjRow<T> qa = adj_row(a, j0 - 1), qb = adj_row(a, j0);
+    for (int m = j0 - 1; m <= j1 + 1; m += 2) {
+        const Row na = load_row(m + 2), nb = load_row(m + 3);
+        const AdjRow<T> nqa = adj_row(a, m + 2), nqb = adj_row(a, m + 3);
+        row(m, ra, qa);
+        row(m + 1, rb, qb);
+        ra = na; rb = nb;
+        qa = nqa; qb = nqb;
     }
+}
+
+template <typename T, bool COR>
+__global__ __launch_bounds__(64) void adj_march_kernel(AdjArgs<T> a)
+{
+    // workgroups go round the 8 XCDs: each takes a contiguous range of strips, whose common
+    // rows then meet in its L2
+    const unsigned gx = gridDim.x, B = gx * gridDim.y, b = blockIdx.x + gx * blockIdx.y;
+    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
+    const unsigned L = xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+    const int by = (int)(L / gx), wg = (int)(L - (unsigned)by * gx);
+    const int c0 = wg * kAdjOwn - 1, j0 = by * a.rows, j1 = min(j0 + a.rows, a.ny);
+    // all its columns, and the rows that its strip's results depend on, interior?
+    if (c0 >= 1 && c0 + 64 <= a.nx - 2 && j0 >= 2 && j1 + 1 <= a.ny - 2)
+        adj_march<T, COR, false>(a, wg, j0, j1);
+    else
+        adj_march<T, COR, true>(a, wg, j0, j1);
 }
 
 // Adds values[g] to lS at the gauge cells: one lane per gauge; the lane of a cell's

@@ -189,7 +189,7 @@ template <int MODE, int L, bool WEIGHTS>
 __global__ __launch_bounds__(kListThreads) void superpose_lists_kernel(SupArgs a)
 {
     extern __shared__ __align__(16) double tile[];   // [nsrc + 1][2 L]; the last row zero
-    constexpr int C = 2 * L, PER = 64 / L;
+    constexpr int C = 2 * L;
     const long long N = (long long)a.gmax * 3 * a.ng;
     const int t = threadIdx.x, li = t % L;
     // MODE 0: first column; MODE 1: first gauge and first sample
