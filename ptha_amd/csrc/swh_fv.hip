@@ -97,16 +97,16 @@ __device__ __forceinline__ double theta_wd(double theta, double d0, double d1, d
     return fmax_(theta * fmin_(1.0, tl), 0.0);
 }
 
-// MC limited gradient (extrapolation_limiting_mod.f90:57-74)
+// MC limited gradient (extrapolation_limiting_mod.f90:57-74): of the two differences, zero
+// where their signs differ, else the smallest in size of their mean and th (>= 0) times each.
+// The reference's form, min or max of the mean and the limited difference by its sign, gives
+// the same values in 20 operations; this takes 12, eight times a cell.
 __device__ __forceinline__ double mc_grad(double lo, double mid, double hi, double th)
 {
     const double a = hi - mid, b = mid - lo;
-    const double sa = copysign(1.0, a), sb = copysign(1.0, b);
-    const double half_sasb = 0.5 * (sa + sb);
-    const double d = fmin_(fabs(a), fabs(b)) * half_sasb * th;
-    const double e = 0.5 * (a + b);
-    const double c = (d == 0.0) ? 0.0 : e;
-    return (d > 0.0) ? fmin_(c, d) : fmax_(c, d);
+    const double m = fmin_(fabs(0.5 * (a + b)), fmin_(fabs(a), fabs(b)) * th);
+    const bool same = (__double2hiint(a) ^ __double2hiint(b)) >= 0;
+    return same ? copysign(m, a) : 0.0;
 }
 
 struct Grad4 {
@@ -257,6 +257,13 @@ __device__ __forceinline__ void cell_sources(const FVArgs<T> &a, int j, const Ce
 // values are loaded one row ahead of their use.
 constexpr int kMOwn = 61;   // owned columns per strip
 
+// v of lane k (the same on every lane)
+__device__ __forceinline__ double lane_value(double v, int k)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                            __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+
 __device__ __forceinline__ double shfl_from_west(double v) { return lane_west(v); }
 __device__ __forceinline__ double shfl_from_east(double v) { return lane_east(v); }
 
@@ -287,7 +294,10 @@ __device__ __forceinline__ void fv_flux_march_body(const FVArgs<T> &a, int rows)
     const bool ew_col = i > 0 && i < a.nx - 1;    // east-west gradients exist in this column
     const Grad4 zero{0.0, 0.0, 0.0, 0.0};
     const long long FP = (long long)a.fpitch * (a.ny + 1), EPn = (long long)a.fpitch * a.ny;
-    const double dle_i = a.dle[gi], inv_ns = 1.0 / (scalar_load(a.dle) * a.half_cfl);   // (the CFL terms' factors)
+    // the CFL terms' factors: of the south edges, and of the west edges of the strip's row
+    // 'lane' (at most 64 rows)
+    const double dle_i = a.dle[gi], inv_ns = 1.0 / (scalar_load(a.dle) * a.half_cfl);
+    const double inv_rows = 1.0 / (a.dbe[min(j0 + lane, a.ny - 1)] * a.half_cfl);
     // rows j0-2, j0-1, j0 and the north-south gradient of row j0-1
     double e_m2, e_m1, e_0;
     const Cell c_m2 = cell_clamped(a, gi, j0 - 2, e_m2);
@@ -326,7 +336,7 @@ __device__ __forceinline__ void fv_flux_march_body(const FVArgs<T> &a, int rows)
             a.fNS[FP + fo] = (T)r.f1;
             a.fNS[2 * FP + fo] = (T)r.f2;
             a.esJ[fo] = r.es_neg;
-            const EdgeOut q = ew_edge(dle_i, 1.0 / (dbe_j * a.half_cfl), w, c_0, g_ew_w, g_ew, e_w, e_0);
+            const EdgeOut q = ew_edge(dle_i, lane_value(inv_rows, j - j0), w, c_0, g_ew_w, g_ew, e_w, e_0);
             a.fEW[fo] = (T)q.f0;
             a.fEW[EPn + fo] = (T)q.f1;
             a.fEW[2 * EPn + fo] = (T)q.f2;
