@@ -282,13 +282,25 @@ __device__ __forceinline__ Cell cell_clamped(const FVArgs<T> &a, int gi, int j, 
     return clip_raw(a, r);
 }
 
+// Workgroup b of the B of a grid goes to XCD b % 8; this gives it a tile of the XCD's own
+// contiguous range, so that tiles that share rows or cache lines meet in one L2: the update reads each row of
+// fluxes for two rows of cells, and a strip of 61 columns ends inside its neighbour's cache
+// lines (60 rk2 steps of 2000 x 1000 in FP64: 19.6 -> 18.3 ms).
+__device__ __forceinline__ unsigned xcd_tile(unsigned b, unsigned B)
+{
+    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
+    return xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+}
+
 template <typename T>
 __device__ __forceinline__ void fv_flux_march_body(const FVArgs<T> &a, int rows)
 {
     const int lane = threadIdx.x;
-    const int i = blockIdx.x * kMOwn - 2 + lane;
+    const unsigned tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    const int by = (int)(tile / gridDim.x), bx = (int)(tile - (unsigned)by * gridDim.x);
+    const int i = bx * kMOwn - 2 + lane;
     const int gi = min(max(i, 0), a.nx - 1);
-    const int j0 = blockIdx.y * rows, j1 = min(j0 + rows, a.ny);
+    const int j0 = by * rows, j1 = min(j0 + rows, a.ny);
     const bool own = lane >= 2 && lane <= 62 && i >= 1 && i < a.nx;
     const bool ns_col = i < a.nx;                 // north-south gradients exist in this column
     const bool ew_col = i > 0 && i < a.nx - 1;    // east-west gradients exist in this column
@@ -537,8 +549,9 @@ __global__ void fv_update_kernel(FVArgs<T> a)
         }
         return;
     }
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = yb;
+    const unsigned tile = xcd_tile(blockIdx.x + gridDim.x * (unsigned)yb, gridDim.x * (unsigned)a.ny);
+    const int j = (int)(tile / gridDim.x), bx = (int)(tile - (unsigned)j * gridDim.x);
+    const int i = bx * blockDim.x + threadIdx.x;
     unsigned long long fixed = 0;
     // with the rk2 average folded in, the step's closing bookkeeping (it does not touch
     // stage_dt, the one scalar this kernel reads; with the scalar pass in this launch,

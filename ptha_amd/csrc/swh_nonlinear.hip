@@ -263,15 +263,30 @@ __device__ __forceinline__ NLCell<T> nl_cell(const NLRaw<T> &w, int r, int ny)
     return c;
 }
 
+// This workgroup's tile (column block bx, row or strip by): workgroup b goes to XCD b % 8, and
+// each XCD gets a contiguous range of the tiles, so that those that share rows or cache lines
+// meet in one L2 (80 steps of 1537 x 1021 in FP64: 9.3 -> 8.75 ms; the momentum update reads
+// three rows of fluxes and state).
+__device__ __forceinline__ void nl_tile(int &bx, int &by)
+{
+    const unsigned gx = gridDim.x, B = gx * gridDim.y, b = blockIdx.x + gx * blockIdx.y;
+    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
+    const unsigned t = xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+    by = (int)(t / gx);
+    bx = (int)(t - (unsigned)by * gx);
+}
+
 template <typename T>
 __global__ __launch_bounds__(64) void nl_flux_march_kernel(NLArgs<T> a, int rows)
 {
     const int nx = a.nx, ny = a.ny, P = a.pitch;
     const int lane = threadIdx.x;
-    const int i = (int)blockIdx.x * kNLOwn - 2 + lane;
+    int bx, by;
+    nl_tile(bx, by);
+    const int i = bx * kNLOwn - 2 + lane;
     const int ci = min(max(i, 0), nx - 1);
     const bool own = lane >= 2 && lane <= kNLOwn + 1 && i < nx;
-    const int j0 = (int)blockIdx.y * rows;
+    const int j0 = by * rows;
     if (j0 >= ny) return;
     const int j1 = min(j0 + rows, ny);
     const int js = j0 == 0 ? 0 : (j0 >= ny - 1 ? j0 - 2 : j0 - 1);
@@ -394,7 +409,9 @@ __device__ __forceinline__ T nl_sign1(T x)
 template <typename T>
 __global__ void nl_momentum_kernel(NLArgs<T> a)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+    int bx, j;
+    nl_tile(bx, j);
+    const int i = bx * blockDim.x + threadIdx.x;
     if (i >= a.nx || j >= a.ny) return;
     const int nx = a.nx, ny = a.ny, P = a.pitch;
     const T *S = a.S, *E = a.E, *UH = a.UH, *VH = a.VH;
