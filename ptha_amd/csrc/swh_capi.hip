@@ -1039,13 +1039,8 @@ int swh_domain_create(const swh_domain_desc *d, swh_domain **out)
     if (h->prec == SWH_PREC_FP64) { h->block_x = 128; h->rows_per_block = 32; h->variant = 1; }
     else { h->block_x = 128; h->rows_per_block = 32; h->variant = 2; }
     if (fv) {
-        // finite volume: rows per wavefront of the flux pass, 8, or 4 where a grid would
-        // have fewer than 4096 wavefronts of 16-byte lanes at 8 (measured on the beach)
-        h->rows_per_block = 8;
-        const int vec = h->prec == SWH_PREC_FP64 ? 2 : 4;
-        const long long waves_x = ((d->nx + vec - 1) / vec + 63) / 64;
-        while (h->rows_per_block > 4 && waves_x * ((d->ny + h->rows_per_block - 1) / h->rows_per_block) < 4096)
-            h->rows_per_block /= 2;
+        // finite volume: rows per wavefront of the flux pass
+        h->rows_per_block = fv_flux_default_rows(d->nx, d->ny, device_cus());
     } else {
         const int vec = (h->variant & 1) ? (h->prec == SWH_PREC_FP64 ? 2 : 4) : 1;
         const long long waves_x = ((d->nx + vec - 1) / vec + 63) / 64;

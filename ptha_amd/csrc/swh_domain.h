@@ -121,6 +121,9 @@ struct swh_domain {
 };
 
 namespace swh {
+
+// rows of a strip of the finite-volume flux pass, from a grid's size (swh_fv.hip)
+int fv_flux_default_rows(int nx, int ny, int cus);
 // One domain%evolve_one_step on the device (leapfrog or rk2), as swh_evolve_one_step.
 int domain_evolve(swh_domain *h, double dt);
 // Re-reads the elevation from the device and rebuilds the leapfrog friction work

@@ -374,7 +374,27 @@ __global__ __launch_bounds__(64) void fv_flux_march_kernel(FVArgs<T> a, int rows
     fv_flux_march_body<T>(a, rows);
 }
 
-int fv_flux_march_rows(int rows) { return rows < 4 ? 4 : (rows > 64 ? 64 : rows); }
+int fv_flux_march_rows(int rows) { return rows < 1 ? 1 : (rows > 64 ? 64 : rows); }
+
+// Rows of a strip of the flux pass, from a grid's size. A strip of r rows costs about r + 1.7
+// (its first cells and gradient), the device holds three of these wavefronts per SIMD, and a
+// last round that is a quarter, half, three quarters full takes about 0.55, 0.7, 0.9 of a
+// full one. Measured per call of 60 rk2 steps for 4 / 6 / 8 / 11 / 16 rows: 2000 x 1000 18.3 /
+// 18.2 / 18.5 / 17.7 / 19.7 ms (3003 wavefronts at 11), 331 x 203 3.8 / 4.2 / 4.6 / 5.2 / 6.3
+// (4 was the least; 3.6 -> 3.1 with one row).
+int fv_flux_default_rows(int nx, int ny, int cus)
+{
+    const double wx = (nx + kMOwn - 1) / kMOwn, cap = 12.0 * cus;
+    int best = 1;
+    double cost = 1e300;
+    for (int r = 1; r <= 32; r++) {
+        const double w = wx * ((ny + r - 1) / r) / cap, q = floor(w), rem = w - q;
+        const double last = rem <= 0.0 ? 0.0 : rem <= 0.25 ? 0.55 : rem <= 0.5 ? 0.7 : rem <= 0.75 ? 0.9 : 1.0;
+        const double t = ((r < ny ? r : ny) + 1.7) * (q + last);
+        if (t < cost) { cost = t; best = r; }
+    }
+    return best;
+}
 
 int fv_flux_grid_blocks(int nx, int ny, int rows)
 {
@@ -383,7 +403,7 @@ int fv_flux_grid_blocks(int nx, int ny, int rows)
 }
 
 // capacity of the per-block maxima: the grid of the shortest strips
-int fv_flux_blocks(int nx, int ny) { return fv_flux_grid_blocks(nx, ny, 4); }
+int fv_flux_blocks(int nx, int ny) { return fv_flux_grid_blocks(nx, ny, 1); }
 
 // ---- pass 3: one block: boundary-flux sums (domain_mod.f90:1483-1499), step choice,
 // time and flux-integral bookkeeping (timestepping_alternatives_include.f90:31-50) ----
