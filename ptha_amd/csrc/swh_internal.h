@@ -427,7 +427,7 @@ struct FVArgs {
     // with avgS and a stage boundary after the update: the pre-average UH of columns 1
     // and nx-2 ([2][ny]) then VH of rows 1 and ny-2 ([2][nx]), which the boundary reads
     T *ring = nullptr;
-    // flux pass: rows per wavefront of the column-marching kernel (4..64)
+    // flux pass: rows per wavefront of the column-marching kernel (1..64)
     int flux_rows = 8;
     // nesting flux integrals of this stage (x += nest_dt * flux on each strip cell),
     // done by extra blocks of the update launch: null or nest_dt == 0: none
