@@ -250,7 +250,7 @@ __device__ __forceinline__ T mom_face(const LFArgs<T> &a, T ch, T cg, T f, T len
 //    they waited behind the next row's state).
 // In FP32 with Coriolis a row of five levels is 245 vector operations (384 before) in the
 // INNER loop. Measured per step: 12 sources of 1200 x 1200 in FP32 49 -> 42.5 us, 32 sources
-// 123 -> 100, 1 source 7.6 -> 5.8; 512 sources see swh_batch_create. FP64: 12 sources 99 -> 64,
+// 123 -> 100, 1 source 7.6 -> 5.8; 512 sources 1.67 -> 1.45 ms. FP64: 12 sources 99 -> 64,
 // 1 source 11.3 -> 7.5.
 // MX (single grids): max_stage after every step. The running maxima of the NS rows in
 // flight move up a ring beside the levels; a row's are read once, before level 1, and
