@@ -100,13 +100,15 @@ __device__ __forceinline__ double theta_wd(double theta, double d0, double d1, d
 // MC limited gradient (extrapolation_limiting_mod.f90:57-74): of the two differences, zero
 // where their signs differ, else the smallest in size of their mean and th (>= 0) times each.
 // The reference's form, min or max of the mean and the limited difference by its sign, gives
-// the same values in 20 operations; this takes 12, eight times a cell.
+// the same values in 20 operations; this takes 13, eight times a cell. Where the signs differ
+// the smaller difference times zero is returned: the reference's NaN (inf * 0) between infinite
+// differences of both signs.
 __device__ __forceinline__ double mc_grad(double lo, double mid, double hi, double th)
 {
     const double a = hi - mid, b = mid - lo;
-    const double m = fmin_(fabs(0.5 * (a + b)), fmin_(fabs(a), fabs(b)) * th);
+    const double w = fmin_(fabs(a), fabs(b)), m = fmin_(fabs(0.5 * (a + b)), w * th);
     const bool same = (__double2hiint(a) ^ __double2hiint(b)) >= 0;
-    return same ? copysign(m, a) : 0.0;
+    return same ? copysign(m, a) : w * 0.0;
 }
 
 struct Grad4 {
