@@ -11,6 +11,7 @@
 
 #include "swh_domain.h"
 #include "swh_launch.h"
+#include "swh_rules.h"
 
 namespace swh {
 
@@ -2815,8 +2816,10 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
     const int TE = superpose_event_tile();
     const int Kpad = (b->nsrc + 3) / 4 * 4;
     const long long ncol = summary == SWH_SUPERPOSE_SERIES ? (long long)b->gmax * 3 * b->ng : b->ng;
-    // as lists of each event's sources (few of all of them), or a dense weight matrix
-    const bool lists = superpose_lists_fit(b->nsrc, n_events, event_ptr[n_events], event_w != nullptr);
+    // as lists of each event's sources, or a dense weight matrix
+    const bool maxima = summary != SWH_SUPERPOSE_SERIES;
+    const bool lists = superpose_lists_fit(b->nsrc, b->ng, maxima ? std::max(ns_all, 1) : b->gmax, n_events,
+                                           event_ptr[n_events], event_w != nullptr, maxima);
     // events per launch: bounded device output (<= 2^28 doubles) and weight matrix
     const long long row = lists ? ncol : std::max<long long>(ncol, Kpad);
     long long chunk = std::max<long long>(TE, ((1LL << 28) / row) / TE * TE);
@@ -2937,7 +2940,7 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
         a.X = b->d_gval; a.slot_stride = (long long)b->gmax * 3 * b->ng;
         a.nsrc = b->nsrc; a.ng = b->ng; a.gmax = b->gmax;
         a.W = d_w; a.Kpad = Kpad; a.E = E; a.scale = d_scale; a.nvalid = d_nv; a.msl = msl;
-        a.s_chunk = 16; a.s_max = std::min(smax, b->gmax);
+        a.s_chunk = kSupChunk; a.s_max = std::min(smax, b->gmax);
         a.out = d_out;
         a.M = d_m;
         if (lists) {

@@ -335,7 +335,6 @@ hipError_t launch_add_scaled(T *E, const T *fE, int pitch, int i0, int i1, int j
 
 // rows of the event tile (W, scale and nvalid must hold a multiple of it)
 int superpose_event_tile();
-bool superpose_lists_fit(int nsrc, long long n_events, long long entries, bool weights);
 hipError_t launch_superpose_lists(const SupArgs &a, int mode, hipStream_t s);
 hipError_t launch_superpose(const SupArgs &a, int mode, hipStream_t s);
 // flags[slot] = 1 where the slot's series (slot_stride values each) holds a non-finite

@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "swh_internal.h"
+#include "swh_rules.h"
 
 namespace swh {
 
@@ -21,8 +22,8 @@ namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTE = 64;  // events per block tile (2 x 2 waves of 32 x 32)
-constexpr int kTN = 64;  // columns per block tile
+constexpr int kTE = kSupTE;   // events per block tile (2 x 2 waves of 32 x 32)
+constexpr int kTN = kSupTN;   // columns per block tile
 
 // seen: a value that *p has held
 __device__ __forceinline__ void atomic_max_f64(double *p, double v, double seen)
@@ -320,25 +321,6 @@ hipError_t launch_superpose(const SupArgs &a, int mode, hipStream_t s)
                                a);
     }
     return hipGetLastError();
-}
-
-// lanes per event of the list kernel (0: the sources' rows do not fit in LDS)
-static int list_lanes(int nsrc)
-{
-    const long long lds = 160 * 1024;
-    return (nsrc + 1LL) * 256 <= lds ? 16 : (nsrc + 1LL) * 128 <= lds ? 8 : 0;
-}
-
-// Whether events with 'entries' list entries in all are taken from lists: while they name
-// less than 0.7 of all event-source pairs (0.4 with weights, which are loaded per entry); the
-// matrix product takes events by 64. Kernel ms of 4096 events' maxima from 512 sources, 600
-// samples, 64 gauges: dense 8.4; lists 0.87 / 1.4 / 3.1 / 5.0 at a share of 0.02 /
-// 0.075 / 0.25 / 0.5, with weights 0.99 / 1.9 / 4.5 / 8.6; 300 events 2.0 against 0.21 at 0.075;
-// the series of 48 events, 301 samples, 48 gauges: 0.155 against 0.06.
-bool superpose_lists_fit(int nsrc, long long n_events, long long entries, bool weights)
-{
-    const double pairs = (double)((n_events + kTE - 1) / kTE * kTE) * nsrc;
-    return list_lanes(nsrc) > 0 && entries < (weights ? 0.4 : 0.7) * pairs;
 }
 
 template <int MODE, int L, bool WEIGHTS>
