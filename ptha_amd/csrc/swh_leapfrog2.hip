@@ -12,7 +12,7 @@
 // UH from memory); each lane owns one column and marches up a strip of rows. At
 // row m it forms step 1 at row m (stage, UH) and m-1 (VH), then step 2 at row m-1
 // (stage, UH) and m-2 (VH), and writes row m-2. East/west neighbours come
-// from the adjacent lanes (lane moves, no LDS tile, no barriers); the
+// from the adjacent lanes (lane moves or permutes, no LDS tile, no barriers); the
 // stencil reaches one column each way per step, which the 3 halo lanes cover.
 // Rows below/above the strip are recomputed by the strip itself (3 extra rows).
 #include <atomic>
@@ -32,6 +32,13 @@ __device__ __forceinline__ void step1_cell(const LFArgs<T> &a, const T *__restri
 // a.bf.ey > 0 (single grid): the first a.bf.ey rows of workgroups take the boundary-flux
 // sums of both steps (the second from UH/VH one step ahead on the lines) and write
 // nothing else.
+// Neighbours come by lane moves, except in FP32 with friction or depths of the moving surface,
+// where the permutes suit better (they leave the vector pipe): us a step at 2048 x 2048 with
+// permutes / moves, FP32 friction 26.5 / 27.6, FP32 moving depths 18.7 / 19.2, truely linear
+// 18.2 / 18.3, FP64 25.7 / 25.0; 400 x 400 FP64 6.2 / 5.9. Row coefficients are vector loads here: through the scalar cache (scalar_load) they
+// are waited for in the row that uses them, or a row ahead take registers; at 1024 x 1024 in
+// FP64 with friction 15.0 / 16.6 / 18.4 us a step as vector loads / scalar / scalar a row ahead.
+// (4096 x 4096, where a wavefront is seldom waited for, is 6 % faster with scalar loads.)
 template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool PF>
 __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
 {
@@ -42,6 +49,7 @@ __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
         });
         return;
     }
+    constexpr bool kMoves = sizeof(T) == 8 || (TL && !FRIC);   // neighbours by lane moves (else permutes)
     int bx, by, bz;
     lf2_tile(a.lf2_order, a.lf2_group, a.bf.ey, bx, by, bz);
     const int lane = threadIdx.x & 63;
@@ -62,6 +70,8 @@ __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
     T *__restrict__ Co = KAHAN ? a.Co + so : nullptr;
     T *__restrict__ UHo = a.UHo + so;
     T *__restrict__ VHo = a.VHo + so;
+    const auto east = [](T v) { if constexpr (kMoves) return shl1(v); else return __shfl_down(v, 1); };
+    const auto west_of = [](T v) { if constexpr (kMoves) return shr1(v); else return __shfl_up(v, 1); };
     const bool west = col == 0;                          // UH(i-1) clamps to UH(0) (include.f90:319-322)
     // per-lane constants: edge lengths and where the column updates
     const T dle_i = a.rc.dle[min(max(col, 0), a.nx)];
@@ -85,12 +95,12 @@ __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
         vh0_p = VH[o];
         uh0_p = UH[o];
         e_p = a.E[o];
-        vh0_p_r = shl1(vh0_p);
+        vh0_p_r = east(vh0_p);
         // every lane takes part in a shuffle (a lane that skips it leaves its neighbour
         // reading an inactive lane), then the western edge keeps its own value
-        const T uh0_p_sh = shr1(uh0_p);
+        const T uh0_p_sh = west_of(uh0_p);
         uh0_p_l = west ? uh0_p : uh0_p_sh;
-        e_p_r = shl1(e_p);
+        e_p_r = east(e_p);
     }
 
     // the loads of one row (lane 0 also reads its own west neighbour's UH)
@@ -119,9 +129,9 @@ __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
         }
         const RowCo<T> q = row_co(a, m);
         // UH(i-1): from the lane to the west; lane 0 has none and reads it itself
-        const T uh0_sh = shr1(uh0);
+        const T uh0_sh = west_of(uh0);
         const T uh0_l = west ? uh0 : (lane == 0 ? uh0_mem : uh0_sh);
-        const T vh0_r = shl1(vh0), e_r = shl1(e);
+        const T vh0_r = east(vh0), e_r = east(e);
         // VH of the row below, clamped to row 0 at the southern edge (include.f90:295-308)
         const T vhb = m > 0 ? vh0_p : vh0, vhb_r = m > 0 ? vh0_p_r : vh0_r;
         // friction work: UH at row m (and m-1 from the last row), VH at row m-1 (and m-2)
@@ -136,24 +146,24 @@ __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
         T s1, c1;
         stage_cell<T, KAHAN>(col_int && q.interior, q.sa, dle_i, q.dbe_lo, q.dbe_hi, s0, c0, uh0, uh0_l, vh0, vhb, s1,
                              c1);
-        const T s1_r = shl1(s1);
-        const T c1_r = KAHAN ? shl1(c1) : T(0);
+        const T s1_r = east(s1);
+        const T c1_r = KAHAN ? east(c1) : T(0);
         const T uh1 = mom_u<T, KAHAN, COR, FRIC, TL, LINF>(a, col_mom && q.valid, q.cu, q.fu, dle_ip1, fw_u1, uh0, s1,
                                                             c1, s1_r, c1_r, e, e_r, vhb, vhb_r, vh0, vh0_r);
-        const T uh1_sh = shr1(uh1);
+        const T uh1_sh = west_of(uh1);
         const T uh1_l = west ? uh1 : uh1_sh;
         // step 1: VH at row m-1
         const T vh1 = mom_v<T, KAHAN, COR, FRIC, TL, LINF>(a, col_mom && q_p.valid, q_p.cv, q_p.fv, q_p.dbe_hi, fw_v1,
                                                             vh0_p, s1_p, c1_p, s1, c1, e_p, e, uh0_p, uh0_p_l, uh0,
                                                             uh0_l);
-        const T vh1_r = shl1(vh1);
+        const T vh1_r = east(vh1);
         // step 2: stage and UH at row m-1 (VH of row m-2 clamped to row 0 at the southern edge)
         const T vhb1 = m - 1 > 0 ? vh1_pp : vh1, vhb1_r = m - 1 > 0 ? vh1_pp_r : vh1_r;
         T s2, c2;
         stage_cell<T, KAHAN>(col_int && q_p.interior, q_p.sa, dle_i, q_p.dbe_lo, q_p.dbe_hi, s1_p, c1_p, uh1_p,
                              uh1_p_l, vh1, vhb1, s2, c2);
-        const T s2_r = shl1(s2);
-        const T c2_r = KAHAN ? shl1(c2) : T(0);
+        const T s2_r = east(s2);
+        const T c2_r = KAHAN ? east(c2) : T(0);
         const T uh2 = mom_u<T, KAHAN, COR, FRIC, TL, LINF>(a, col_mom && q_p.valid, q_p.cu, q_p.fu, dle_ip1, fw_u2,
                                                             uh1_p, s2, c2, s2_r, c2_r, e_p, e_p_r, vhb1, vhb1_r, vh1,
                                                             vh1_r);

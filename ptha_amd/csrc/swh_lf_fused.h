@@ -31,13 +31,13 @@ __device__ __forceinline__ RowCo<T> row_co(const LFArgs<T> &a, int r)
 {
     const int rc = min(max(r, 0), a.ny - 1);
     RowCo<T> q;
-    q.sa = scalar_load(a.rc.sa + rc);
-    q.cu = scalar_load(a.rc.cu + rc);
-    q.cv = scalar_load(a.rc.cv + rc);
-    q.fu = scalar_load(a.rc.fu + rc);
-    q.fv = scalar_load(a.rc.fv + rc);
-    q.dbe_lo = scalar_load(a.rc.dbe + rc);
-    q.dbe_hi = scalar_load(a.rc.dbe + rc + 1);
+    q.sa = a.rc.sa[rc];
+    q.cu = a.rc.cu[rc];
+    q.cv = a.rc.cv[rc];
+    q.fu = a.rc.fu[rc];
+    q.fv = a.rc.fv[rc];
+    q.dbe_lo = a.rc.dbe[rc];
+    q.dbe_hi = a.rc.dbe[rc + 1];
     q.interior = r > 0 && r < a.ny - 1;
     q.valid = r >= 0 && r < a.ny - 1;
     return q;
