@@ -548,6 +548,14 @@ int bf_flush(swh_domain *h)
     return SWH_OK;
 }
 
+// The end of a call that took fused launches, also one that failed with rc: the steps that were
+// taken count, so their boundary fluxes and their end time do.
+int fused_end(swh_domain *h, int rc)
+{
+    const int rc_flush = bf_flush(h);
+    return rc ? rc : rc_flush;
+}
+
 // how many of the next ns steps update max_U
 int maxq_due(const swh_domain *h, int ns)
 {
@@ -1315,11 +1323,7 @@ int swh_evolve_steps(swh_domain *h, double timestep, int32_t nsteps)
         if (ns && fused_ok(h, timestep, ns)) {
             rc = leapfrog_fused_any(h, timestep, ns);
             k += ns;
-            if (!rc && k >= nsteps) rc = bf_flush(h);
-            if (rc) {
-                h->lb_pending = 0;
-                return rc;
-            }
+            if (rc || k >= nsteps) return fused_end(h, rc);
             continue;
         }
         if ((rc = bf_flush(h))) return rc;
@@ -1875,9 +1879,7 @@ int swh_evolve_record_gauges_schedule(swh_domain *h, double timestep, int32_t ns
             q++;
         }
     }
-    if (!rc) rc = bf_flush(h);
-    h->lb_pending = 0;
-    return rc;
+    return fused_end(h, rc);
 }
 
 int swh_checkpoint_save(swh_domain *h, int32_t slot)
