@@ -556,33 +556,31 @@ int fused_end(swh_domain *h, int rc)
     return rc ? rc : rc_flush;
 }
 
-// how many of the next ns steps update max_U
-int maxq_due(const swh_domain *h, int ns)
+// how many of ns steps after the first n update max_U
+int maxq_due(const swh_domain *h, int ns, long long n)
 {
     int due = 0;
     if (h->maxq_mask)
-        for (int k = 0; k < ns; k++) due += (h->nsteps + k) % h->maxq_freq == 0;
+        for (int k = 0; k < ns; k++) due += (n + k) % h->maxq_freq == 0;
     return due;
 }
 
-// Whether the next ns leapfrog steps can run as one fused launch: as two_step_ok, for ns
-// steps, and max_U not due in any of them, or max_stage alone due in all (which the launch
-// keeps; a mixture would need its masks in the loop).
-bool fused_ok(const swh_domain *h, double dt, int ns)
+// Whether ns leapfrog steps from time t, after the first n, can run as one fused launch: as
+// two_step_ok, for ns steps, and max_U not due in any of them, or max_stage alone due in all
+// (which the launch keeps; a mixture would need its masks in the loop).
+bool fused_ok(const swh_domain *h, double dt, int ns, double t, long long n)
 {
     if (!h->two_step || h->rows2 || !h->d_lb || h->bc_mask || h->n_nest_strips ||
         h->nx <= 2 * h->n_ext || h->ny <= 2 * h->n_ext)
         return false;
     if (h->method == SWH_METHOD_LLPNF && (!h->truely_linear || !h->fw_ready)) return false;
-    if (h->f_on) {
-        double t = h->time;
+    if (h->f_on)
         for (int k = 0; k < ns; k++) {
             const double t_half = t + dt * 0.5;
             if (forcing_fraction(h, t_half, dt) != 0.0) return false;
             t = t_half + 0.5 * dt;
         }
-    }
-    const int due = maxq_due(h, ns);
+    const int due = maxq_due(h, ns, n);
     if (due && (due != ns || h->maxq_mask != SWH_MAXQ_MAX_STAGE)) return false;
     return (long long)h->pitch * h->ny < (1LL << 31);
 }
@@ -595,6 +593,24 @@ bool fused_ok(const swh_domain *h, double dt, int ns)
 int fused_depth(long long left)
 {
     return left % 3 == 0 && left > 0 ? 3 : 0;
+}
+
+// Whether the run of fused launches of ns steps that can be taken from now, with 'left' steps to
+// go, is long enough (fused_least_run). window(k, t): can its k'th launch, at time t, be taken?
+template <typename Window>
+bool fused_worth(const swh_domain *h, double dt, int ns, long long left, Window window)
+{
+    const bool simple = h->method == SWH_METHOD_LINEAR && h->truely_linear;
+    const bool fp64 = h->prec == SWH_PREC_FP64, due = maxq_due(h, ns, h->nsteps) > 0;
+    const long long most = std::min<long long>(left / ns, kFusedRunMost);
+    long long run = 0;
+    for (double t = h->time; run < most && window(run, t); run++)
+        for (int i = 0; i < ns; i++) t = (t + dt * 0.5) + 0.5 * dt;
+    // steps to the call's end, or to the next update of max_U, which may end a pair
+    const long long f = h->maxq_freq, n = h->nsteps;
+    const long long stretch = h->maxq_mask ? std::min(left, (f - n % f) % f + 1) : left;
+    const bool odd = stretch % 2 != 0 && run % 2 != 0;
+    return run && run >= fused_least_run((long long)h->nx * h->ny, simple, fp64, due, odd);
 }
 
 int fused_strip_rows(const swh_domain *h, int ns)
@@ -631,7 +647,7 @@ int leapfrog_fused(swh_domain *h, double dt, int ns, int level = 0)
     a.src_fast = 0;
     a.maxq_mask = 0; a.mx = (T *)h->mx; a.t_after = T(0); a.arrival_stage = T(0);
     a.lf2_order = 1; a.lf2_group = 1;
-    if (maxq_due(h, ns)) a.mx_levels = (1 << ns) - 1;
+    if (maxq_due(h, ns, h->nsteps)) a.mx_levels = (1 << ns) - 1;
     // the boundary fluxes: this launch's lines into one buffer, the sums of the launch before
     // it from the other
     const size_t half = (size_t)24 * h->lb_len;
@@ -1320,7 +1336,8 @@ int swh_evolve_steps(swh_domain *h, double timestep, int32_t nsteps)
     for (int k = 0; k < nsteps;) {
         int rc;
         const int ns = timestep > 0.0 && h->d_lb ? fused_depth(nsteps - k) : 0;
-        if (ns && fused_ok(h, timestep, ns)) {
+        const auto ok = [&](long long m, double t) { return fused_ok(h, timestep, ns, t, h->nsteps + m * ns); };
+        if (ns && (h->lb_pending ? ok(0, h->time) : fused_worth(h, timestep, ns, nsteps - k, ok))) {
             rc = leapfrog_fused_any(h, timestep, ns);
             k += ns;
             if (rc || k >= nsteps) return fused_end(h, rc);
@@ -1824,8 +1841,9 @@ int swh_evolve_record_gauges_schedule(swh_domain *h, double timestep, int32_t ns
             sample_steps[q] > (int64_t)INT32_MAX)
             return fail(SWH_EINVAL, "sample steps must be >= 0 and strictly increasing");
     if (h->gsamples + nsamples > h->gmax) return fail(SWH_ESTATE, "gauge sample buffer too small");
-    // steps in pairs wherever two_step_ok allows, whatever the sample spacing: a sample
-    // due between the two steps of a pair is taken one step ahead by the pair itself
+    // fused launches where they follow one another for long enough, else pairs wherever
+    // two_step_ok allows, whatever the sample spacing: a sample due between the two steps of a
+    // pair is taken one step ahead by the pair itself
     const long long last = sample_steps[nsamples - 1];
     long long n = 0;
     int q = 0, rc = SWH_OK;
@@ -1836,32 +1854,43 @@ int swh_evolve_record_gauges_schedule(swh_domain *h, double timestep, int32_t ns
     // fused launches take one sample inside where the scheme allows (truely-linear 'linear',
     // gauges that fit the lanes), else they end at it
     const bool inside = h->method == SWH_METHOD_LINEAR && h->truely_linear && h->ng > 0 && h->d_gij;
+    const bool fit = inside && gauges_fit_rows(h, fused_strip_rows(h, 3));
+    // Can a fused launch of ns steps start m steps into the call, at time t and after the domain's
+    // first nst steps, with sample s next? level: the step after which it takes it (0: none inside).
+    const auto window = [&](long long m, int s, int ns, double t, long long nst, int &level) {
+        level = 0;
+        if (!fused_ok(h, timestep, ns, t, nst)) return false;
+        if (s >= nsamples || sample_steps[s] > m + ns) return true;
+        if (s + 1 < nsamples && sample_steps[s + 1] <= m + ns) return false;
+        if (fit && !maxq_due(h, ns, nst)) level = (int)(sample_steps[s] - m);
+        return level || sample_steps[s] == m + ns;
+    };
     while (!rc && n < last) {
-        int ns = h->d_lb ? fused_depth(last - n) : 0;
-        if (ns) {
-            const auto count = [&](int m) {   // samples due in the next m steps
-                int due = 0;
-                while (q + due < nsamples && sample_steps[q + due] <= n + m) due++;
-                return due;
-            };
-            if (ns == 5 && count(5) > 1) ns = 3;
-            const int due = count(ns);
-            int level = due ? (int)(sample_steps[q] - n) : 0;
-            const bool at_end = due == 1 && level == ns;
-            if (due && !(due == 1 && inside && !maxq_due(h, ns) && gauges_fit_rows(h, fused_strip_rows(h, ns)))) {
-                if (!at_end) ns = 0;
-                level = 0;
+        const int ns = h->d_lb ? fused_depth(last - n) : 0;
+        int level = 0;
+        bool go = false;
+        if (ns && h->lb_pending) {
+            go = window(n, q, ns, h->time, h->nsteps, level);
+        } else if (ns) {
+            int s = q;
+            go = fused_worth(h, timestep, ns, last - n, [&](long long k, double t) {
+                int l;
+                const long long m = n + k * ns;
+                if (!window(m, s, ns, t, h->nsteps + k * ns, l)) return false;
+                if (k == 0) level = l;
+                while (s < nsamples && sample_steps[s] <= m + ns) s++;
+                return true;
+            });
+        }
+        if (go) {
+            rc = leapfrog_fused_any(h, timestep, ns, level);
+            n += ns;
+            if (level) q++;
+            if (!rc && q < nsamples && sample_steps[q] == n) {
+                rc = swh_gauges_sample(h);
+                q++;
             }
-            if (ns && fused_ok(h, timestep, ns)) {
-                rc = leapfrog_fused_any(h, timestep, ns, level);
-                n += ns;
-                if (level) q++;
-                if (!rc && q < nsamples && sample_steps[q] == n) {
-                    rc = swh_gauges_sample(h);
-                    q++;
-                }
-                continue;
-            }
+            continue;
         }
         if ((rc = bf_flush(h))) break;
         const bool mid = q < nsamples && sample_steps[q] == n + 1;

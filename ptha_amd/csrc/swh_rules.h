@@ -56,4 +56,32 @@ inline bool superpose_lists_fit(int nsrc, int ng, long long samples, long long n
     return lists < dense;
 }
 
+// How many fused launches of three leapfrog steps have to follow one another on a single grid
+// to be begun: the last one's boundary-flux sums cost a launch of their own (8 us), and each
+// launch gains less than that over what it replaces where the grid is small. 'simple': truely
+// linear without friction, whose rows are the shortest; 'due': max_stage after every step (it
+// replaces three single steps, else one and a half pairs); 'odd': an odd number of launches in a
+// stretch of an odd number of steps (to the call's end or the next update of max_U), of which pairs
+// would leave a single step, which costs more than half a pair. In an even stretch a lone launch
+// would leave such a step itself. Gain per launch in us, FP64 / FP32, max_stage not due: 8 x 6
+// simple 1.6 / 1.6; 150 x 150 3.7 / 5.2, friction 3.4 / 6.1; 400 x 400 5.2 / 7.0, 1.0 / 6.7;
+// 1024 x 1024 6.4 / 5.2, 3.8 / -0.2; 2048 x 2048 18 / 15, 31 / 10. Due: 8 x 6 3.7 / 3.7,
+// 0.7 / 1.3; 150 x 150 4.0 / 5.2, 1.3 / 3.1; 400 x 400 12 / 9.4, 5.2 / 6.1; 700 x 500 19 / 17,
+// 13 / 14.
+constexpr int kFusedRunMost = 5;   // the most that is asked for
+
+inline int fused_least_run(long long cells, bool simple, bool fp64, bool due, bool odd)
+{
+    if (due) {
+        if (cells >= 300000) return 1;
+        if (cells >= 100000) return simple ? 1 : 2;
+        return simple || (!fp64 && cells >= 10000) ? 2 : 5;
+    }
+    if (odd && cells >= 300000) return 1;
+    if (cells >= 3000000) return 2;
+    if (simple) return cells >= 100000 ? 2 : cells >= 10000 ? 3 : 4;
+    if (fp64) return cells >= 300000 ? 3 : 5;
+    return cells >= 10000 && cells < 800000 ? 2 : 5;
+}
+
 }  // namespace swh

@@ -17,6 +17,10 @@ extern "C" int lists_fit(int nsrc, int ng, long long samples, long long events, 
 {
     return swh::superpose_lists_fit(nsrc, ng, samples, events, entries, w != 0, maxima != 0);
 }
+extern "C" int least_run(long long cells, int simple, int fp64, int due, int odd)
+{
+    return swh::fused_least_run(cells, simple != 0, fp64 != 0, due != 0, odd != 0);
+}
 """
 
 
@@ -34,6 +38,7 @@ def rules(tmp_path_factory):
     lib = ctypes.CDLL(so)
     q = ctypes.c_longlong
     lib.lists_fit.argtypes = [ctypes.c_int, ctypes.c_int, q, q, q, ctypes.c_int, ctypes.c_int]
+    lib.least_run.argtypes = [q] + 4 * [ctypes.c_int]
     return lib
 
 
@@ -80,3 +85,31 @@ def test_events_take_the_faster_route(rules, row):
 def test_lists_only_where_they_fit(rules):
     assert rules.lists_fit(1279, 64, 100, 100, 1000, 0, 1)
     assert not rules.lists_fit(1280, 64, 100, 100, 1000, 0, 1)
+
+
+# cells, truely linear without friction, FP64, max_stage after every step; us of a fused launch of
+# three steps, of what it replaces (three single steps, or one and a half pairs), and of the
+# extra launch that ends a run
+RUNS = [
+    (48, 1, 1, 0, 9.9, 11.5, 7.2), (48, 1, 1, 1, 10.5, 14.2, 7.4), (48, 0, 0, 1, 12.9, 14.2, 7.1),
+    (2000, 1, 1, 0, 10.5, 13.0, 7.6), (2000, 0, 1, 0, 14.4, 16.9, 7.7), (2000, 0, 0, 1, 12.9, 14.5, 8.3),
+    (22500, 1, 1, 0, 10.5, 14.2, 8.2), (22500, 1, 1, 1, 11.4, 15.4, 8.3), (22500, 0, 1, 0, 12.3, 14.2, 7.8),
+    (22500, 0, 0, 0, 12.3, 18.4, 7.8), (22500, 0, 1, 1, 15.6, 16.9, 8.0), (160000, 1, 1, 0, 12.6, 17.8, 7.8),
+    (160000, 1, 0, 0, 10.2, 17.2, 7.8), (160000, 1, 1, 1, 13.5, 25.9, 7.8), (160000, 0, 1, 0, 15.0, 17.5, 7.9),
+    (160000, 0, 0, 0, 15.3, 22.0, 7.4), (160000, 0, 1, 1, 21.3, 26.5, 8.2), (350000, 1, 1, 0, 13.8, 22.6, 7.4),
+    (350000, 0, 1, 1, 23.4, 36.1, 7.6), (1048576, 1, 1, 0, 24.8, 31.3, 8.5), (1048576, 1, 0, 0, 19.1, 24.4, 8.5),
+    (1048576, 0, 1, 0, 40.1, 43.9, 9.2), (1048576, 0, 0, 1, 36.2, 58.3, 8.6), (1650000, 0, 0, 0, 25.8, 30.1, 8.6),
+    (4194304, 1, 0, 0, 39.0, 54.1, 8.6), (4194304, 0, 1, 0, 106.8, 137.5, 8.2), (4194304, 0, 0, 1, 76.4, 167.7, 8.1),
+]
+
+
+@pytest.mark.parametrize("row", RUNS)
+def test_runs_of_fused_launches_pay(rules, row):
+    cells, simple, fp64, due, fused, replaced, flush = row
+    least = rules.least_run(cells, simple, fp64, due, 0)
+    assert 1 <= least <= 5
+    assert least * fused + flush <= 1.08 * least * replaced
+    # and those that pay clearly are taken
+    assert 5 * fused + flush > 0.75 * 5 * replaced or least < 5
+    assert due or least > 1      # (a lone launch in an even stretch leaves a single step)
+    assert rules.least_run(cells, simple, fp64, due, 1) <= least
