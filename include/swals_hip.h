@@ -424,6 +424,11 @@ int swh_probe_valu(int32_t fp64, int32_t blocks, int32_t iters, int32_t reps, do
 int swh_probe_math(int32_t n, const double *x, const double *y, const double *t, double *pow_dev, double *sin_dev,
                    double *pow_host, double *sin_host);
 
+/* Check utility (no counterpart in the reference): the dispersive solve of this domain uses the
+ * smaller work buffer (7 planes, the same bits) that swh_dispersion_enable takes where the
+ * usual one of 13 planes cannot be allocated. Before swh_dispersion_enable. */
+int swh_probe_dispersion_compact(swh_domain *h);
+
 /* ---------------------------------------------------------------------------
  * Multidomain nesting on one GPU (multidomain_mod.f90, nested_grid_comms_mod.f90).
  *

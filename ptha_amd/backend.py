@@ -135,6 +135,7 @@ SYMBOLS = [
     ("swh_adjoint_run", ctypes.c_int, [ctypes.c_void_p, _D, _I32, _I32, _PD]),
     ("swh_probe_copy", ctypes.c_int, [ctypes.c_int64, _I32, _PD]),
     ("swh_probe_valu", ctypes.c_int, [_I32, _I32, _I32, _I32, _PD, _PD]),
+    ("swh_probe_dispersion_compact", ctypes.c_int, [ctypes.c_void_p]),
     ("swh_probe_math", ctypes.c_int, [_I32, _PD, _PD, _PD, _PD, _PD, _PD, _PD]),
     ("swh_md_create", ctypes.c_int, [_I32, ctypes.POINTER(ctypes.c_void_p), _PD, _PI32, _PI32,
                                      ctypes.POINTER(ctypes.c_void_p)]),

@@ -794,6 +794,7 @@ int dispersion_solve(swh_domain *h, int buf, int rhs_up, int estimate, double ft
     a.msl = (T)h->msl; a.dlon = (T)h->disp_dlon; a.dlat = (T)h->disp_dlat;
     a.td1 = (T)h->disp_td1; a.td2 = (T)h->disp_td2;
     a.cell = h->leapfrog() ? 0 : 1;
+    a.compact = h->disp_compact;
     a.sc = ftime_on_device ? h->sc : nullptr;
     a.t_fwd = ftime;
     // no extrapolation before three levels: ten times the iterations instead (:1267-1291)
@@ -1577,6 +1578,30 @@ int swh_gauges_download(swh_domain *h, double *values, double *times, int32_t *n
     return SWH_OK;
 }
 
+// the work buffer of the dispersive solve: the smaller one where the other doesn't fit
+static int dispersion_work(swh_domain *h)
+{
+    if (!h->disp_compact) {
+        const size_t bytes = dispersion_work_elems(h->nx, h->ny, false) * h->esz;
+        if (hipMalloc(&h->dwork, bytes) == hipSuccess) {
+            SWH_HIP(hipMemset(h->dwork, 0, bytes));
+            return SWH_OK;
+        }
+        (void)hipGetLastError();
+        h->dwork = nullptr;
+        h->disp_compact = 1;
+    }
+    return dmalloc(&h->dwork, dispersion_work_elems(h->nx, h->ny, true) * h->esz);
+}
+
+int swh_probe_dispersion_compact(swh_domain *h)
+{
+    if (!h) return fail(SWH_EINVAL, "null argument");
+    if (h->disp_on) return fail(SWH_ESTATE, "swh_probe_dispersion_compact goes before swh_dispersion_enable");
+    h->disp_compact = 1;
+    return SWH_OK;
+}
+
 int swh_dispersion_enable(swh_domain *h, double dlon, double dlat, double td1, double td2, int32_t niter)
 {
     if (!h) return fail(SWH_EINVAL, "null argument");
@@ -1590,7 +1615,7 @@ int swh_dispersion_enable(swh_domain *h, double dlon, double dlat, double td1, d
         int rc = dmalloc(&h->dlast, 3 * P);
         if (!rc) rc = dmalloc(&h->drhs, 2 * P);
         for (int k = 0; k < 3 && !rc; k++) rc = dmalloc(&h->dq[k], 2 * P);
-        if (!rc) rc = dmalloc(&h->dwork, dispersion_work_elems(h->nx, h->ny) * h->esz);
+        if (!rc) rc = dispersion_work(h);
         if (!rc) rc = dmalloc((void **)&h->d_qt, 3 * sizeof(double));
         if (rc) return rc;
         h->disp_on = 1;

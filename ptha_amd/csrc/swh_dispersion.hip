@@ -163,7 +163,10 @@ __global__ void disp_extrapolate_kernel(DispArgs<T> a)
 // beforehand (div_by). 700 x 517
 // FP64: a walk takes 40 us (VH) to 53 us (UH), the elimination of both directions 92 us
 // once per solve, where a sweep with a lane doing all of a line's work took 1170 and 1360
-// us; a dispersive step (two iterations) 480 us, 5.2 ms before.
+// us; a dispersive step (two iterations) 480 us, 5.2 ms before. The matrices take six values per
+// element and direction: 13 planes of work with the right-hand side, where the sweeps needed
+// 4. Where those don't fit in device memory, the directions share a place (7 planes) and every
+// iteration eliminates anew: the same bits, a step of 0.65 ms takes 1.09.
 constexpr int kTile = 32;    // tile of the transposing kernels
 
 template <typename T>
@@ -182,14 +185,16 @@ struct DispWork {
     T *b;              // right-hand side and solution of the sweep at hand
 };
 
+// (compact: one direction's matrices at a time, in the same place)
 template <typename T>
-__host__ __device__ inline DispWork<T> disp_work(T *W, long long n)
+__host__ __device__ inline DispWork<T> disp_work(const DispArgs<T> &a)
 {
+    const long long n = (long long)a.nx * a.ny, second = a.compact ? 0 : n;
     DispWork<T> w;
-    w.c4[0] = (Coef4<T> *)W;
-    w.c4[1] = w.c4[0] + n;
+    w.c4[0] = (Coef4<T> *)a.W;
+    w.c4[1] = w.c4[0] + second;
     w.c2[0] = (Coef2<T> *)(w.c4[1] + n);
-    w.c2[1] = w.c2[0] + n;
+    w.c2[1] = w.c2[0] + second;
     w.b = (T *)(w.c2[1] + n);
     return w;
 }
@@ -304,15 +309,15 @@ __device__ __forceinline__ T vh_rhs(const DispArgs<T> &a, int i, int j)
                             T(1) / Rdlon_j * (a.UH[o] - a.UH[o - 1])));
 }
 
-// The matrices of both directions, a thread per cell: blockIdx.z 0 the rows of UH
+// The matrices, a thread per cell, of direction dir0 + blockIdx.z: 0 the rows of UH
 // (j = 1 .. ny-2, transposed to element i, line j through LDS), 1 the columns of VH.
 template <typename T>
-__global__ __launch_bounds__(256) void disp_coef_kernel(DispArgs<T> a)
+__global__ __launch_bounds__(256) void disp_coef_kernel(DispArgs<T> a, int dir0)
 {
-    const DispWork<T> w = disp_work(a.W, (long long)a.nx * a.ny);
+    const DispWork<T> w = disp_work(a);
     const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile;
     const int tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;
-    if (blockIdx.z == 1) {
+    if (dir0 + (int)blockIdx.z == 1) {
         const int i = i0 + tx;
         for (int r = ty; r < kTile; r += 256 / kTile) {
             const int j = j0 + r;
@@ -405,7 +410,7 @@ __global__ __launch_bounds__(kWalkThreads) void disp_factor_kernel(DispArgs<T> a
 {
     constexpr int C = 8;
     __shared__ T buf[2][C][3][kLines];
-    const DispWork<T> w = disp_work(a.W, (long long)a.nx * a.ny);
+    const DispWork<T> w = disp_work(a);
     const int dir = (int)blockIdx.x >= blocks_uh ? 1 : 0, lane = threadIdx.x % kLines;
     const int sub = (threadIdx.x & 63) / kLines;   // which of the elements that a loader takes at once
     const int n = dir ? a.ny : a.nx, lines = dir ? a.nx : a.ny;
@@ -483,10 +488,10 @@ __global__ __launch_bounds__(kWalkThreads) void disp_factor_kernel(DispArgs<T> a
 // the reciprocals of the eliminated diagonals (NaN where div_by does not hold), a thread
 // per cell: off the elimination's chain
 template <typename T>
-__global__ __launch_bounds__(256) void disp_recip_kernel(DispArgs<T> a)
+__global__ __launch_bounds__(256) void disp_recip_kernel(DispArgs<T> a, int dir0)
 {
-    const DispWork<T> w = disp_work(a.W, (long long)a.nx * a.ny);
-    const int dir = blockIdx.z, n = dir ? a.ny : a.nx, lines = dir ? a.nx : a.ny;
+    const DispWork<T> w = disp_work(a);
+    const int dir = dir0 + (int)blockIdx.z, n = dir ? a.ny : a.nx, lines = dir ? a.nx : a.ny;
     const int line = 1 + blockIdx.x * 256 + threadIdx.x, k = blockIdx.y;
     if (line > lines - 2 || k >= n - 1) return;
     Coef4<T> *q = w.c4[dir] + (long long)k * lines + line;
@@ -499,7 +504,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void disp_uh_rhs_kernel(DispArgs<T> a)
 {
     __shared__ T tile[kTile][kTile + 1];
-    T *b = disp_work(a.W, (long long)a.nx * a.ny).b;
+    T *b = disp_work(a).b;
     const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile;
     const int tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;
     for (int r = ty; r < kTile; r += 256 / kTile) {
@@ -518,7 +523,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void disp_uh_put_kernel(DispArgs<T> a)
 {
     __shared__ T tile[kTile][kTile + 1];
-    const T *b = disp_work(a.W, (long long)a.nx * a.ny).b;
+    const T *b = disp_work(a).b;
     const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile;
     const int tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;
     for (int r = ty; r < kTile; r += 256 / kTile) {
@@ -537,7 +542,7 @@ __global__ __launch_bounds__(256) void disp_vh_rhs_kernel(DispArgs<T> a)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
     if (i < 1 || i > a.nx - 2) return;
-    disp_work(a.W, (long long)a.nx * a.ny).b[(long long)j * a.nx + i] = vh_rhs(a, i, j);
+    disp_work(a).b[(long long)j * a.nx + i] = vh_rhs(a, i, j);
 }
 
 __device__ __forceinline__ int exponent_of(double x) { return __builtin_amdgcn_frexp_exp(x); }
@@ -728,19 +733,23 @@ hipError_t launch_dispersion(const DispArgs<T> &a, int make_rhs, int extrapolate
     if (extrapolate) hipLaunchKernelGGL(disp_extrapolate_kernel<T>, grid, block, 0, s, a);
     const dim3 tiles((a.nx + kTile - 1) / kTile, (a.ny + kTile - 1) / kTile);
     const int bu = (a.ny - 2 + kLines - 1) / kLines, bv = (a.nx - 2 + kLines - 1) / kLines;
-    const DispWork<T> w = disp_work(a.W, (long long)a.nx * a.ny);
-    if (niter > 0) {
-        // the elevation may have changed since the last solve: the matrices anew
-        hipLaunchKernelGGL(disp_coef_kernel<T>, dim3(tiles.x, tiles.y, 2), block, 0, s, a);
-        hipLaunchKernelGGL(disp_factor_kernel<T>, dim3(bu + bv), dim3(kWalkThreads), 0, s, a, bu);
-        const int most = std::max(a.nx, a.ny);
-        hipLaunchKernelGGL(disp_recip_kernel<T>, dim3((most + 255) / 256, most, 2), block, 0, s, a);
-    }
+    const DispWork<T> w = disp_work(a);
+    // the matrices of 'dirs' directions from dir0, eliminated
+    const auto matrices = [&](int dir0, int dirs) {
+        const int rows = dir0 ? 0 : bu, columns = dir0 + dirs > 1 ? bv : 0, most = std::max(a.nx, a.ny);
+        hipLaunchKernelGGL(disp_coef_kernel<T>, dim3(tiles.x, tiles.y, dirs), block, 0, s, a, dir0);
+        hipLaunchKernelGGL(disp_factor_kernel<T>, dim3(rows + columns), dim3(kWalkThreads), 0, s, a, rows);
+        hipLaunchKernelGGL(disp_recip_kernel<T>, dim3((most + 255) / 256, most, dirs), block, 0, s, a, dir0);
+    };
+    // (the elevation may have changed since the last solve)
+    if (niter > 0 && !a.compact) matrices(0, 2);
     for (int it = 0; it < niter; it++) {
+        if (a.compact) matrices(0, 1);
         hipLaunchKernelGGL(disp_uh_rhs_kernel<T>, tiles, block, 0, s, a);
         hipLaunchKernelGGL(disp_walk_kernel<T>, dim3(bu), dim3(kWalkThreads), 0, s, (const Coef4<T> *)w.c4[0],
                            (const Coef2<T> *)w.c2[0], w.b, a.nx, a.ny, w.b, (long long)a.ny);
         hipLaunchKernelGGL(disp_uh_put_kernel<T>, tiles, block, 0, s, a);
+        if (a.compact) matrices(1, 1);
         hipLaunchKernelGGL(disp_vh_rhs_kernel<T>, grid, block, 0, s, a);
         hipLaunchKernelGGL(disp_walk_kernel<T>, dim3(bv), dim3(kWalkThreads), 0, s, (const Coef4<T> *)w.c4[1],
                            (const Coef2<T> *)w.c2[1], w.b, a.ny, a.nx, a.VH, (long long)a.pitch);
@@ -748,7 +757,7 @@ hipError_t launch_dispersion(const DispArgs<T> &a, int make_rhs, int extrapolate
     return hipGetLastError();
 }
 
-size_t dispersion_work_elems(int nx, int ny) { return 13 * (size_t)nx * ny; }
+size_t dispersion_work_elems(int nx, int ny, bool compact) { return (compact ? 7 : 13) * (size_t)nx * ny; }
 
 template hipError_t launch_dispersion<double>(const DispArgs<double> &, int, int, int, hipStream_t);
 template hipError_t launch_dispersion<float>(const DispArgs<float> &, int, int, int, hipStream_t);

@@ -33,7 +33,7 @@ struct swh_domain {
     void *ring = nullptr;
     // dispersion (leapfrog methods, midpoint/rk2/euler): stored UH/VH/elevation, right-hand side, three
     // extrapolation levels (oldest first) with their times, tridiagonal work
-    int disp_on = 0, disp_iter = 2;
+    int disp_on = 0, disp_iter = 2, disp_compact = 0;   // (compact: the smaller work buffer)
     double disp_td1 = 0.0, disp_td2 = -1.0, disp_dlon = 1.0, disp_dlat = 1.0;
     void *dlast = nullptr, *drhs = nullptr, *dq[3] = {}, *dwork = nullptr;
     double *d_qt = nullptr;   // level times (device: finite-volume times live there)

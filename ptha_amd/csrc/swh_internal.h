@@ -286,6 +286,7 @@ struct DispArgs {
     const double *dbe, *dle;
     T msl, dlon, dlat, td1, td2;
     int cell;                    // 1: cell-centred (finite-volume) form, 0: staggered
+    int compact;                 // W holds one direction's matrices at a time
     const DevScalars *sc;        // forward time of the extrapolation from sc->time when set
     double t_fwd;                // else this forward time
 };
@@ -293,7 +294,7 @@ struct DispArgs {
 // from Y0..Y2; then niter tridiagonal iterations (rows of UH, then columns of VH)
 template <typename T>
 hipError_t launch_dispersion(const DispArgs<T> &a, int make_rhs, int extrapolate, int niter, hipStream_t s);
-size_t dispersion_work_elems(int nx, int ny);
+size_t dispersion_work_elems(int nx, int ny, bool compact);
 // shift the level times down one and record the new level's time (sc->time or t_host)
 hipError_t launch_dispersion_qt_append(double *qt, const DevScalars *sc, double t_host, hipStream_t s);
 
