@@ -372,11 +372,13 @@ int swh_batch_launch_counts(swh_batch *b, int64_t *launches, int64_t *source_lau
 int swh_batch_set_launch(swh_batch *b, int32_t block_x, int32_t rows_per_block, int32_t variant);
 /* Launch-shape autotuner (no counterpart in the reference): times every one-step shape
  * (variant 0..15 x block_x {64,128,256} x rows {16,32,64}) and every fused shape (2..5
- * steps per launch x block_x {64,128,256} x rows {32,64,128,256} x tile order:
+ * steps per launch x block_x {64,128,256} x rows {31,63,127,255} x tile order:
  * hardware, or XCD order with sources interleaved in groups of 16) over reps repeats
  * of the next launch on this batch's own grid and running sources, keeps the fastest
  * per cell-update, and returns it in best[3] = {block_x, rows_per_block, variant} with
- * its time per step.
+ * its time per step. A batch whose shape was never set or tuned chooses rows and depth for
+ * each launch; it goes on doing so unless a fixed shape is more than 2 % faster (best[] is
+ * then the shape that its launches have now).
  * The state and step count are left as they were. Needs the step counts and the
  * elevation set. */
 int swh_batch_autotune(swh_batch *b, double dt, int32_t reps, int32_t *best, double *best_ms);

@@ -2388,13 +2388,24 @@ int batch_evolve(swh_batch *b, double dt, int nsteps)
     return SWH_OK;
 }
 
+// the tile order's bits of a launch variant
+int launch_order_bits(int xcd_order, int group)
+{
+    int lg = 0;
+    while ((1 << lg) < group) lg++;
+    return xcd_order ? 64 | (lg << 7) : 0;
+}
+
 // Launch-shape autotuner: times every candidate shape on the batch's own grid and
 // sources by repeating the next step(s) (each launch reads the current buffer and
 // writes the other, which the next real step overwrites), so the state and step count
 // are unchanged. One-step shapes: variant 0..15 x block_x {64,128,256} x rows
 // {16,32,64}; then the fused kernels: 2..5 steps per launch x block_x x rows
 // {31,...,255} x tile order (hardware, or XCD order with sources interleaved in groups
-// of 16), compared per cell-update of the running sources.
+// of 16), compared per cell-update of the running sources. A batch that still chooses height
+// and depth for each launch (rows_per_block 0) keeps doing so unless a fixed shape is more than
+// 2 % faster now: it also follows the sources as they end. (One source of 300 x 300 in FP32:
+// 2.5 us a step, the fastest fixed shape 8.6; 64 of 1200 x 1200 in FP64 295 and 305.)
 template <typename T, bool KAHAN>
 int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *best_ms)
 {
@@ -2413,6 +2424,7 @@ int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *bes
     double bms = 1e300;   // ms per step of n_active sources
     int bb = b->block_x, br = b->rows_per_block, bv = b->variant | (b->src_fast << 3) | (b->two_step << 4);
     int bx_order = b->xcd_order, b_group = b->src_group, b_fuse = b->fuse;
+    const int bx_order0 = bx_order, b_group0 = b_group;
     // one launch of depth D (1..5) over the sources with D or more steps left
     auto launch = [&](int D, int nD) -> int {
         if (D == 1) return batch_launch<T, KAHAN>(b, a, fric_mode, nD, c);
@@ -2435,6 +2447,13 @@ int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *bes
         ms_out = (double)ms / reps / D * ((double)n_active / nD);
         return SWH_OK;
     };
+    const bool can2 = fric_mode <= 1 && (long long)g->plane_elems() < (1LL << 31);
+    const bool automatic = b->rows_per_block == 0;
+    const int auto_bx = b->block_x, auto_v = b->variant, auto_sf = b->src_fast, auto_two = b->two_step, auto_fuse = b->fuse;
+    const int auto_D = can2 && auto_two ? std::max(2, std::min(5, batch_depth(b, n_active))) : 1;
+    const int auto_rows = automatic ? batch_rows(b, n_active, auto_D) : 0;
+    double auto_ms = 1e300;
+    if (automatic) rc = timed(auto_D, auto_ms);
     const int rws1[3] = {16, 32, 64};
     for (int v = 0; v < 16 && rc == SWH_OK; v++)
         for (int ib = 0; ib < 3 && rc == SWH_OK; ib++)
@@ -2444,7 +2463,7 @@ int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *bes
                 rc = timed(1, ms);
                 if (!rc && ms < bms) { bms = ms; bb = bxs[ib]; br = rws1[ir]; bv = v; }
             }
-    if (!rc && fric_mode <= 1 && (long long)g->plane_elems() < (1LL << 31)) {
+    if (!rc && can2) {
         // fused kernels with the next row's loads in flight
         const int v1 = bv | 2;
         b->variant = v1 & 7; b->src_fast = (v1 >> 3) & 1;
@@ -2466,18 +2485,25 @@ int batch_autotune(swh_batch *b, double dt, int reps, int32_t *best, double *bes
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
+    if (automatic && (rc || auto_ms <= 1.02 * bms)) {
+        // (what is returned is the shape that its launches have now)
+        bms = auto_ms;
+        b->block_x = auto_bx; b->rows_per_block = 0; b->variant = auto_v; b->src_fast = auto_sf;
+        b->two_step = auto_two; b->fuse = auto_fuse; b->xcd_order = bx_order0; b->src_group = b_group0;
+        bb = auto_D == 3 ? 64 : auto_bx;
+        br = auto_rows;
+        bv = auto_v | (auto_sf << 3);
+        if (auto_D > 1) bv |= 16 | launch_order_bits(bx_order0, b_group0) | ((auto_D - 2) << 10);
+        if (rc) return rc;
+        if (best) { best[0] = bb; best[1] = br; best[2] = bv; }
+        if (best_ms) *best_ms = bms;
+        return SWH_OK;
+    }
     b->block_x = bb; b->rows_per_block = br; b->variant = bv & 7; b->src_fast = (bv >> 3) & 1;
     b->two_step = (bv >> 4) & 1;
     b->xcd_order = bx_order; b->src_group = b_group;
     b->fuse = b->two_step ? b_fuse : 2;
-    if (b->two_step) {
-        if (bx_order) {
-            int lg = 0;
-            while ((1 << lg) < b_group) lg++;
-            bv |= 64 | (lg << 7);
-        }
-        bv |= (b->fuse - 2) << 10;
-    }
+    if (b->two_step) bv |= launch_order_bits(bx_order, b_group) | ((b->fuse - 2) << 10);
     if (rc) return rc;
     if (best) { best[0] = bb; best[1] = br; best[2] = bv; }
     if (best_ms) *best_ms = bms;

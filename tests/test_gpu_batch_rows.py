@@ -46,3 +46,26 @@ def test_rows_chosen_per_launch(precision, nx, ny, steps):
                         d.evolve_one_step(dt)
                 assert np.array_equal(b.get_source(k), d.U[:3]), k
                 assert np.array_equal(b.gauge_series(k), d.gauge_series()[1]), k
+
+
+def test_autotune_keeps_what_no_fixed_shape_beats():
+    """One small source needs strips of a few rows, shorter than any fixed shape that the tuner
+    tries (2.5 us a step against 8.6 with the best of those): tuning must not leave
+    the batch slower than it found it. The allowance, a half, covers the clock's scatter."""
+    print("CASE autotune keeps automatic", flush=True)
+    nx, ny, dt, steps = 300, 300, 3.0, 300
+    rng = np.random.default_rng(1)
+    elev = -4000.0 + 500.0 * rng.random((ny, nx))
+    with UnitSourceBatch(nx, ny, (5.0, 5.0), (150.0, -30.0), 1, precision="fp32k") as b:
+        b.set_elevation(elev)
+        b.set_nsteps(np.array([20 * steps], dtype=np.int32))
+        b.set_source(0, rng.standard_normal((ny, nx)))
+        b.evolve(dt, steps)
+        before = min(b.evolve_timed(dt, steps) for _ in range(4))
+        state = b.get_source(0)
+        (bx, rows, variant), ms = b.autotune(dt)
+        assert np.array_equal(b.get_source(0), state) and ms > 0
+        after = min(b.evolve_timed(dt, steps) for _ in range(4))
+        assert after <= 1.5 * before, (before, after)
+        b.set_launch(bx, rows, variant)   # what is returned is a shape that can be set
+        b.evolve(dt, 3)
