@@ -175,11 +175,8 @@ __device__ __forceinline__ void adj_march(const AdjArgs<T> &a, int wg, int j0, i
 template <typename T, bool COR>
 __global__ __launch_bounds__(64) void adj_march_kernel(AdjArgs<T> a)
 {
-    // workgroups go round the 8 XCDs: each takes a contiguous range of strips, whose common
-    // rows then meet in its L2
-    const unsigned gx = gridDim.x, B = gx * gridDim.y, b = blockIdx.x + gx * blockIdx.y;
-    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
-    const unsigned L = xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+    // each XCD takes a contiguous range of strips, whose common rows then meet in its L2
+    const unsigned gx = gridDim.x, L = xcd_tile(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
     const int by = (int)(L / gx), wg = (int)(L - (unsigned)by * gx);
     const int c0 = wg * kAdjOwn - 1, j0 = by * a.rows, j1 = min(j0 + a.rows, a.ny);
     // all its columns, and the rows that its strip's results depend on, interior?

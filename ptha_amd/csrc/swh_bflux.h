@@ -157,11 +157,9 @@ __device__ void bf_lines(const BfLines &b, int nx, int ny, int pitch, const T *_
 }
 
 // The sums of bf_lines from line buffers [level][side N, E, S, W][len] (the pre-step UH/VH of
-// 'levels' steps that an earlier launch took, at most kBfLevels), by nlb workgroups of
+// 'levels' steps that an earlier launch took, at most kFusedSteps), by nlb workgroups of
 // which this is the k'th: the same split of a side over its workgroups, the same trees and
 // the same bookkeeping, step by step.
-constexpr int kBfLevels = 6;
-
 template <typename T>
 __device__ void bf_sum_lines(const BfLines &b, int nx, int ny, const T *__restrict__ lines, int len_max, int levels,
                              int k, int nlb)
@@ -170,8 +168,8 @@ __device__ void bf_sum_lines(const BfLines &b, int nx, int ny, const T *__restri
     const int q = k & 3, r = k >> 2, nbq = (nlb - q + 3) >> 2;
     const int len = max((q & 1) == 0 ? nx - 2 * ne : ny - 2 * ne, 0);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    __shared__ double wsum[4][kBfLevels][2];
-    __shared__ double st[kBfLevels][4];
+    __shared__ double wsum[4][kFusedSteps][2];
+    __shared__ double st[kFusedSteps][4];
     __shared__ int last;
     for (int l = 0; l < levels; l++) {
         const T *__restrict__ p = lines + (4 * l + q) * len_max;
@@ -189,7 +187,7 @@ __device__ void bf_sum_lines(const BfLines &b, int nx, int ny, const T *__restri
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double *part = b.part + (size_t)k * (2 * kBfLevels);
+        double *part = b.part + (size_t)k * (2 * kFusedSteps);
         for (int l = 0; l < levels; l++) {
             DD x{wsum[0][l][0], wsum[0][l][1]};
             for (int ww = 1; ww < nw; ww++) x = dd_add(x, DD{wsum[ww][l][0], wsum[ww][l][1]});
@@ -210,7 +208,7 @@ __device__ void bf_sum_lines(const BfLines &b, int nx, int ny, const T *__restri
         const int nb = (nlb - qq + 3) >> 2;
         DD x{0.0, 0.0};
         for (int rr = lane; rr < nb; rr += 64) {
-            const double *p = b.part + (size_t)(qq + 4 * rr) * (2 * kBfLevels) + 2 * ll;
+            const double *p = b.part + (size_t)(qq + 4 * rr) * (2 * kFusedSteps) + 2 * ll;
             const double hi = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const double lo = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             x = dd_add(x, DD{hi, lo});

@@ -538,7 +538,7 @@ int bf_flush(swh_domain *h)
     if (!h->lb_pending) return SWH_OK;
     BfLines b = bf_args(h, 256, h->lb_dt, 0.0, 0.0);
     for (int l = 0; l < h->lb_pending; l++) b.t_after[l] = h->lb_t[l];
-    const size_t off = (size_t)(1 - h->lb_cur) * 24 * h->lb_len;
+    const size_t off = (size_t)(1 - h->lb_cur) * kFusedSteps * 4 * h->lb_len;
     const int levels = h->lb_pending;
     h->lb_pending = 0;
     if (h->prec == SWH_PREC_FP64)
@@ -556,56 +556,56 @@ int fused_end(swh_domain *h, int rc)
     return rc ? rc : rc_flush;
 }
 
-// how many of ns steps after the first n update max_U
-int maxq_due(const swh_domain *h, int ns, long long n)
+// how many of a fused launch's steps, after the first n, update max_U
+int maxq_due(const swh_domain *h, long long n)
 {
     int due = 0;
     if (h->maxq_mask)
-        for (int k = 0; k < ns; k++) due += (n + k) % h->maxq_freq == 0;
+        for (int k = 0; k < kFusedSteps; k++) due += (n + k) % h->maxq_freq == 0;
     return due;
 }
 
-// Whether ns leapfrog steps from time t, after the first n, can run as one fused launch: as
-// two_step_ok, for ns steps, and max_U not due in any of them, or max_stage alone due in all
+// Whether a fused launch can take the leapfrog steps from time t, after the first n: as
+// two_step_ok, for its steps, and max_U not due in any of them, or max_stage alone due in all
 // (which the launch keeps; a mixture would need its masks in the loop).
-bool fused_ok(const swh_domain *h, double dt, int ns, double t, long long n)
+bool fused_ok(const swh_domain *h, double dt, double t, long long n)
 {
     if (!h->two_step || h->rows2 || !h->d_lb || h->bc_mask || h->n_nest_strips ||
         h->nx <= 2 * h->n_ext || h->ny <= 2 * h->n_ext)
         return false;
     if (h->method == SWH_METHOD_LLPNF && (!h->truely_linear || !h->fw_ready)) return false;
     if (h->f_on)
-        for (int k = 0; k < ns; k++) {
+        for (int k = 0; k < kFusedSteps; k++) {
             const double t_half = t + dt * 0.5;
             if (forcing_fraction(h, t_half, dt) != 0.0) return false;
             t = t_half + 0.5 * dt;
         }
-    const int due = maxq_due(h, ns, n);
-    if (due && (due != ns || h->maxq_mask != SWH_MAXQ_MAX_STAGE)) return false;
+    const int due = maxq_due(h, n);
+    if (due && (due != kFusedSteps || h->maxq_mask != SWH_MAXQ_MAX_STAGE)) return false;
     return (long long)h->pitch * h->ny < (1LL << 31);
 }
 
-// Steps of the next fused launch with 'left' steps to go (0: take a step or a pair
-// another way): three where the rest divides by three, so that what is left over goes first
-// and the last launch's sums are the only ones flushed. Deeper launches move less memory, but
+// Whether a fused launch may be next with 'left' steps to go: where the rest divides by its
+// three, so that what is left over goes first and the last launch's sums are the only ones
+// flushed. Deeper launches move less memory, but
 // walk more rows per strip: four or five FP32 steps take 5.8-7.1 us a step against 5.6 at
 // 1024^2, 3.9-4.3 against 3.4 at 400^2, and 11.9-13.2 against 12.7 at 2048^2.
-int fused_depth(long long left)
+bool fused_turn(const swh_domain *h, long long left)
 {
-    return left % 3 == 0 && left > 0 ? 3 : 0;
+    return h->d_lb && left > 0 && left % kFusedSteps == 0;
 }
 
-// Whether the run of fused launches of ns steps that can be taken from now, with 'left' steps to
-// go, is long enough (fused_least_run). window(k, t): can its k'th launch, at time t, be taken?
+// Whether the run of fused launches that can be taken from now, with 'left' steps to go, is
+// long enough (fused_least_run). window(k, t): can its k'th launch, at time t, be taken?
 template <typename Window>
-bool fused_worth(const swh_domain *h, double dt, int ns, long long left, Window window)
+bool fused_worth(const swh_domain *h, double dt, long long left, Window window)
 {
     const bool simple = h->method == SWH_METHOD_LINEAR && h->truely_linear;
-    const bool fp64 = h->prec == SWH_PREC_FP64, due = maxq_due(h, ns, h->nsteps) > 0;
-    const long long most = std::min<long long>(left / ns, kFusedRunMost);
+    const bool fp64 = h->prec == SWH_PREC_FP64, due = maxq_due(h, h->nsteps) > 0;
+    const long long most = std::min<long long>(left / kFusedSteps, kFusedRunMost);
     long long run = 0;
     for (double t = h->time; run < most && window(run, t); run++)
-        for (int i = 0; i < ns; i++) t = (t + dt * 0.5) + 0.5 * dt;
+        for (int i = 0; i < kFusedSteps; i++) t = (t + dt * 0.5) + 0.5 * dt;
     // steps to the call's end, or to the next update of max_U, which may end a pair
     const long long f = h->maxq_freq, n = h->nsteps;
     const long long stretch = h->maxq_mask ? std::min(left, (f - n % f) % f + 1) : left;
@@ -613,15 +613,15 @@ bool fused_worth(const swh_domain *h, double dt, int ns, long long left, Window 
     return run && run >= fused_least_run((long long)h->nx * h->ny, simple, fp64, due, odd);
 }
 
-int fused_strip_rows(const swh_domain *h, int ns)
+int fused_strip_rows(const swh_domain *h)
 {
-    return fused_rows(h->nx, h->ny, 1, ns, 65 - 2 * ns, h->prec == SWH_PREC_FP64 ? 128 : 256);
+    return fused_rows(h->nx, h->ny, 1, kFusedSteps, 65 - 2 * kFusedSteps, h->prec == SWH_PREC_FP64 ? 128 : 256);
 }
 
-// ns leapfrog steps in one launch (swh_leapfrog_sg.hip). level (1..ns, or 0): also record
+// kFusedSteps leapfrog steps in one launch (swh_leapfrog_sg.hip). level (1.., or 0): also record
 // a gauge sample after that step.
 template <typename T, bool KAHAN>
-int leapfrog_fused(swh_domain *h, double dt, int ns, int level = 0)
+int leapfrog_fused(swh_domain *h, double dt, int level)
 {
     if (h->rc_dt != dt) {
         int rc = build_rc<T>(h, dt);
@@ -643,14 +643,14 @@ int leapfrog_fused(swh_domain *h, double dt, int ns, int level = 0)
     a.lin_fric_mult = (T)(1.0 / (1.0 + dt * h->lfc));
     a.fric_power = T(0);
     a.bc_mask = 0; a.bc_stage = T(0);
-    a.rows_per_block = fused_strip_rows(h, ns);
+    a.rows_per_block = fused_strip_rows(h);
     a.src_fast = 0;
     a.maxq_mask = 0; a.mx = (T *)h->mx; a.t_after = T(0); a.arrival_stage = T(0);
     a.lf2_order = 1; a.lf2_group = 1;
-    if (maxq_due(h, ns, h->nsteps)) a.mx_levels = (1 << ns) - 1;
+    if (maxq_due(h, h->nsteps)) a.mx_levels = (1 << kFusedSteps) - 1;
     // the boundary fluxes: this launch's lines into one buffer, the sums of the launch before
     // it from the other
-    const size_t half = (size_t)24 * h->lb_len;
+    const size_t half = (size_t)kFusedSteps * 4 * h->lb_len;
     a.lb_len = h->lb_len;
     a.lb_out = (T *)h->d_lb + h->lb_cur * half;
     a.bf.n_ext = h->n_ext;
@@ -660,8 +660,8 @@ int leapfrog_fused(swh_domain *h, double dt, int ns, int level = 0)
         a.lb_in = (const T *)h->d_lb + (1 - h->lb_cur) * half;
         a.lb_levels = h->lb_pending;
     }
-    double t = h->time, t_prev = t, ends[6];
-    for (int k = 0; k < ns; k++) {
+    double t = h->time, t_prev = t, ends[kFusedSteps];
+    for (int k = 0; k < kFusedSteps; k++) {
         t_prev = t;
         t = (t + dt * 0.5) + 0.5 * dt;
         ends[k] = t;
@@ -674,24 +674,24 @@ int leapfrog_fused(swh_domain *h, double dt, int ns, int level = 0)
         a.g_time = h->d_gtime + h->gsamples;
         a.g_t = ends[level - 1];
     }
-    SWH_HIP(launch_leapfrog_sg<T, KAHAN>(a, h->coriolis, fric_mode, h->truely_linear, h->lfc != 0.0, ns, h->stream));
+    SWH_HIP(launch_leapfrog_sg<T, KAHAN>(a, h->coriolis, fric_mode, h->truely_linear, h->lfc != 0.0, h->stream));
     if (level) h->gsamples++;
-    for (int k = 0; k < ns; k++) h->lb_t[k] = ends[k];
-    h->lb_pending = ns;
+    for (int k = 0; k < kFusedSteps; k++) h->lb_t[k] = ends[k];
+    h->lb_pending = kFusedSteps;
     h->lb_dt = dt;
     h->lb_cur = 1 - h->lb_cur;
     h->cur = o;
     h->time = t;
     h->dt_last_update = dt;
     h->evolve_step_dt = t - t_prev;
-    h->nsteps += ns;
+    h->nsteps += kFusedSteps;
     return SWH_OK;
 }
 
-int leapfrog_fused_any(swh_domain *h, double dt, int ns, int level = 0)
+int leapfrog_fused_any(swh_domain *h, double dt, int level = 0)
 {
-    return h->prec == SWH_PREC_FP64 ? leapfrog_fused<double, false>(h, dt, ns, level)
-                                    : leapfrog_fused<float, true>(h, dt, ns, level);
+    return h->prec == SWH_PREC_FP64 ? leapfrog_fused<double, false>(h, dt, level)
+                                    : leapfrog_fused<float, true>(h, dt, level);
 }
 
 template <typename T>
@@ -794,7 +794,7 @@ int dispersion_solve(swh_domain *h, int buf, int rhs_up, int estimate, double ft
     a.msl = (T)h->msl; a.dlon = (T)h->disp_dlon; a.dlat = (T)h->disp_dlat;
     a.td1 = (T)h->disp_td1; a.td2 = (T)h->disp_td2;
     a.cell = h->leapfrog() ? 0 : 1;
-    a.compact = h->disp_compact;
+    a.second = h->disp_compact ? 0 : (long long)h->nx * h->ny;
     a.sc = ftime_on_device ? h->sc : nullptr;
     a.t_fwd = ftime;
     // no extrapolation before three levels: ten times the iterations instead (:1267-1291)
@@ -1138,10 +1138,10 @@ int swh_domain_create(const swh_domain_desc *d, swh_domain **out)
     // line workgroups: at most 4 ceil(max(nx, ny) / 64) wanted, in rows at most
     // ceil(nx / 64) workgroups wide
     h->bf_cap = 4 * ((std::max(nx, ny) + 63) / 64) + (nx + 63) / 64;
-    A((void **)&h->d_bfpart, sizeof(double) * 12 * (size_t)h->bf_cap);
+    A((void **)&h->d_bfpart, sizeof(double) * 2 * kFusedSteps * (size_t)h->bf_cap);
     if (h->method == SWH_METHOD_LINEAR || h->method == SWH_METHOD_LLPNF) {
         h->lb_len = std::max(nx, ny) - 2 * n_ext;
-        A(&h->d_lb, (size_t)2 * 6 * 4 * h->lb_len * h->esz);
+        A(&h->d_lb, (size_t)2 * kFusedSteps * 4 * h->lb_len * h->esz);
     }
     A((void **)&h->d_work, sizeof(double) * (2 * (size_t)ny + 16));
     if (rc) {
@@ -1336,11 +1336,11 @@ int swh_evolve_steps(swh_domain *h, double timestep, int32_t nsteps)
     if (nsteps < 0) return fail(SWH_EINVAL, "nsteps must be >= 0");
     for (int k = 0; k < nsteps;) {
         int rc;
-        const int ns = timestep > 0.0 && h->d_lb ? fused_depth(nsteps - k) : 0;
-        const auto ok = [&](long long m, double t) { return fused_ok(h, timestep, ns, t, h->nsteps + m * ns); };
-        if (ns && (h->lb_pending ? ok(0, h->time) : fused_worth(h, timestep, ns, nsteps - k, ok))) {
-            rc = leapfrog_fused_any(h, timestep, ns);
-            k += ns;
+        const auto ok = [&](long long m, double t) { return fused_ok(h, timestep, t, h->nsteps + m * kFusedSteps); };
+        if (timestep > 0.0 && fused_turn(h, nsteps - k) &&
+            (h->lb_pending ? ok(0, h->time) : fused_worth(h, timestep, nsteps - k, ok))) {
+            rc = leapfrog_fused_any(h, timestep);
+            k += kFusedSteps;
             if (rc || k >= nsteps) return fused_end(h, rc);
             continue;
         }
@@ -1879,37 +1879,37 @@ int swh_evolve_record_gauges_schedule(swh_domain *h, double timestep, int32_t ns
     // fused launches take one sample inside where the scheme allows (truely-linear 'linear',
     // gauges that fit the lanes), else they end at it
     const bool inside = h->method == SWH_METHOD_LINEAR && h->truely_linear && h->ng > 0 && h->d_gij;
-    const bool fit = inside && gauges_fit_rows(h, fused_strip_rows(h, 3));
-    // Can a fused launch of ns steps start m steps into the call, at time t and after the domain's
-    // first nst steps, with sample s next? level: the step after which it takes it (0: none inside).
-    const auto window = [&](long long m, int s, int ns, double t, long long nst, int &level) {
+    const bool fit = inside && gauges_fit_rows(h, fused_strip_rows(h));
+    // Can a fused launch start m steps into the call, at time t and after the domain's first
+    // nst steps, with sample s next? level: the step after which it takes it (0: none inside).
+    const auto window = [&](long long m, int s, double t, long long nst, int &level) {
         level = 0;
-        if (!fused_ok(h, timestep, ns, t, nst)) return false;
-        if (s >= nsamples || sample_steps[s] > m + ns) return true;
-        if (s + 1 < nsamples && sample_steps[s + 1] <= m + ns) return false;
-        if (fit && !maxq_due(h, ns, nst)) level = (int)(sample_steps[s] - m);
-        return level || sample_steps[s] == m + ns;
+        if (!fused_ok(h, timestep, t, nst)) return false;
+        if (s >= nsamples || sample_steps[s] > m + kFusedSteps) return true;
+        if (s + 1 < nsamples && sample_steps[s + 1] <= m + kFusedSteps) return false;
+        if (fit && !maxq_due(h, nst)) level = (int)(sample_steps[s] - m);
+        return level || sample_steps[s] == m + kFusedSteps;
     };
     while (!rc && n < last) {
-        const int ns = h->d_lb ? fused_depth(last - n) : 0;
+        const bool turn = fused_turn(h, last - n);
         int level = 0;
         bool go = false;
-        if (ns && h->lb_pending) {
-            go = window(n, q, ns, h->time, h->nsteps, level);
-        } else if (ns) {
+        if (turn && h->lb_pending) {
+            go = window(n, q, h->time, h->nsteps, level);
+        } else if (turn) {
             int s = q;
-            go = fused_worth(h, timestep, ns, last - n, [&](long long k, double t) {
+            go = fused_worth(h, timestep, last - n, [&](long long k, double t) {
                 int l;
-                const long long m = n + k * ns;
-                if (!window(m, s, ns, t, h->nsteps + k * ns, l)) return false;
+                const long long m = n + k * kFusedSteps;
+                if (!window(m, s, t, h->nsteps + k * kFusedSteps, l)) return false;
                 if (k == 0) level = l;
-                while (s < nsamples && sample_steps[s] <= m + ns) s++;
+                while (s < nsamples && sample_steps[s] <= m + kFusedSteps) s++;
                 return true;
             });
         }
         if (go) {
-            rc = leapfrog_fused_any(h, timestep, ns, level);
-            n += ns;
+            rc = leapfrog_fused_any(h, timestep, level);
+            n += kFusedSteps;
             if (level) q++;
             if (!rc && q < nsamples && sample_steps[q] == n) {
                 rc = swh_gauges_sample(h);
@@ -2074,7 +2074,7 @@ struct swh_batch {
     // rows_most
     int block_x = 256, rows_per_block = 0, rows_most = 256, variant = 2, src_fast = 0;
     int two_step = 0;              // two fused steps per launch where possible
-    int fuse = 2;                  // most fused steps per launch (2..4) where two_step is on
+    int fuse = 2;                  // most fused steps per launch of a set shape, where two_step is on
     int xcd_order = 0;             // two-step launches: XCD-aware tile order
     int src_group = 1;             // ... interleaving the tiles of this many sources
     // step-kernel launches so far: count, sources summed over launches, and source
@@ -2532,14 +2532,14 @@ int swh_batch_create(const swh_domain_desc *desc, int32_t nsources, swh_batch **
         return rc;
     }
     b->nsrc = nsources;
-    // default launch: fused steps (batch_depth), 2-wave blocks, XCD tile order with sources in
+    // default launch: fused steps by batch_depth, 2-wave blocks, XCD tile order with sources in
     // groups of 16, strips of up to 256 / 128 rows (the fastest shapes measured on the
     // 512-source 1200^2 workload; shorter strips where a launch has few sources: batch_rows;
     // swh_batch_autotune refines it per batch)
     b->block_x = 256; b->two_step = 1; b->src_fast = 0;
     b->xcd_order = 1; b->src_group = 16;
-    if (b->g->prec == SWH_PREC_FP64) { b->block_x = 128; b->rows_most = 128; b->variant = 3; b->fuse = 3; }
-    else { b->block_x = 128; b->rows_most = 256; b->variant = 3; b->fuse = 5; }
+    if (b->g->prec == SWH_PREC_FP64) { b->block_x = 128; b->rows_most = 128; b->variant = 3; }
+    else { b->block_x = 128; b->rows_most = 256; b->variant = 3; }
     const size_t bytes = b->g->plane_elems() * b->g->esz * (size_t)nsources;
     const bool kahan = b->g->prec == SWH_PREC_FP32K;
     for (int k = 0; k < 2 && rc == SWH_OK; k++) {
@@ -2941,8 +2941,8 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
         rc = dmalloc((void **)&d_w, sizeof(double) * chunk * Kpad);
         if (!rc && any_flagged) rc = dmalloc((void **)&d_m, sizeof(double) * chunk * Kpad);
     }
-    if (!rc) rc = dmalloc((void **)&d_scale, sizeof(double) * chunk);
-    if (!rc) rc = dmalloc((void **)&d_nv, sizeof(int) * chunk);
+    if (!rc && !lists) rc = dmalloc((void **)&d_scale, sizeof(double) * chunk);
+    if (!rc && !lists) rc = dmalloc((void **)&d_nv, sizeof(int) * chunk);
     if (!rc) rc = dmalloc((void **)&d_out, sizeof(double) * chunk * ncol);
     hipEvent_t t0 = nullptr, t1 = nullptr;
     double total_ms = 0.0;
@@ -3011,8 +3011,9 @@ int swh_batch_superpose(swh_batch *b, int32_t n_events, const int32_t *event_ptr
         }
         if ((!W.empty() &&
              hipMemcpy(d_w, W.data(), sizeof(double) * W.size(), hipMemcpyHostToDevice) != hipSuccess) ||
-            hipMemcpy(d_scale, scale.data(), sizeof(double) * chunk, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(d_nv, nv.data(), sizeof(int) * chunk, hipMemcpyHostToDevice) != hipSuccess ||
+            (d_scale &&
+             hipMemcpy(d_scale, scale.data(), sizeof(double) * chunk, hipMemcpyHostToDevice) != hipSuccess) ||
+            (d_nv && hipMemcpy(d_nv, nv.data(), sizeof(int) * chunk, hipMemcpyHostToDevice) != hipSuccess) ||
             (d_m &&
              hipMemcpy(d_m, M.data(), sizeof(double) * M.size(), hipMemcpyHostToDevice) != hipSuccess)) {
             rc = fail(SWH_EHIP, "superposition upload failed");

@@ -157,13 +157,13 @@ __global__ void disp_extrapolate_kernel(DispArgs<T> a)
 // lines (11 wavefronts on a 700 x 517 grid), so its time is the chain of dependent
 // operations per element. Everything that is not part of that chain is out of it:
 // coefficients and right-hand sides are formed by kernels with a thread per cell (the UH
-// ones transposed through LDS), coefficients are packed so that an element is one or
-// two wide loads, kChunk elements of loads are in flight while the chunk before them is
-// computed, and the division of the back substitution is by a reciprocal formed
-// beforehand (div_by). 700 x 517
-// FP64: a walk takes 40 us (VH) to 53 us (UH), the elimination of both directions 92 us
-// once per solve, where a sweep with a lane doing all of a line's work took 1170 and 1360
-// us; a dispersive step (two iterations) 480 us, 5.2 ms before. The matrices take six values per
+// ones transposed through LDS), coefficients are packed so that an element is one or two
+// wide loads, which wavefronts of their own bring into LDS ahead of the computing one
+// (walk_phases), and the division of the back substitution is by a reciprocal formed
+// beforehand (div_by). 700 x 517 FP64: a walk takes 46 us (53 with 64 lines to a workgroup
+// instead of 16), the elimination of both directions 92 us once per solve, where a sweep with
+// a lane doing all of a line's work took 1170 and 1360 us; a dispersive step (two iterations)
+// 480 us, 5.2 ms before. The matrices take six values per
 // element and direction: 13 planes of work with the right-hand side, where the sweeps needed
 // 4. Where those don't fit in device memory, the directions share a place (7 planes) and every
 // iteration eliminates anew: the same bits, a step of 0.65 ms takes 1.09.
@@ -185,16 +185,15 @@ struct DispWork {
     T *b;              // right-hand side and solution of the sweep at hand
 };
 
-// (compact: one direction's matrices at a time, in the same place)
 template <typename T>
 __host__ __device__ inline DispWork<T> disp_work(const DispArgs<T> &a)
 {
-    const long long n = (long long)a.nx * a.ny, second = a.compact ? 0 : n;
+    const long long n = (long long)a.nx * a.ny;
     DispWork<T> w;
     w.c4[0] = (Coef4<T> *)a.W;
-    w.c4[1] = w.c4[0] + second;
+    w.c4[1] = w.c4[0] + a.second;
     w.c2[0] = (Coef2<T> *)(w.c4[1] + n);
-    w.c2[1] = w.c2[0] + second;
+    w.c2[1] = w.c2[0] + a.second;
     w.b = (T *)(w.c2[1] + n);
     return w;
 }
@@ -742,14 +741,14 @@ hipError_t launch_dispersion(const DispArgs<T> &a, int make_rhs, int extrapolate
         hipLaunchKernelGGL(disp_recip_kernel<T>, dim3((most + 255) / 256, most, dirs), block, 0, s, a, dir0);
     };
     // (the elevation may have changed since the last solve)
-    if (niter > 0 && !a.compact) matrices(0, 2);
+    if (niter > 0 && a.second) matrices(0, 2);
     for (int it = 0; it < niter; it++) {
-        if (a.compact) matrices(0, 1);
+        if (!a.second) matrices(0, 1);
         hipLaunchKernelGGL(disp_uh_rhs_kernel<T>, tiles, block, 0, s, a);
         hipLaunchKernelGGL(disp_walk_kernel<T>, dim3(bu), dim3(kWalkThreads), 0, s, (const Coef4<T> *)w.c4[0],
                            (const Coef2<T> *)w.c2[0], w.b, a.nx, a.ny, w.b, (long long)a.ny);
         hipLaunchKernelGGL(disp_uh_put_kernel<T>, tiles, block, 0, s, a);
-        if (a.compact) matrices(1, 1);
+        if (!a.second) matrices(1, 1);
         hipLaunchKernelGGL(disp_vh_rhs_kernel<T>, grid, block, 0, s, a);
         hipLaunchKernelGGL(disp_walk_kernel<T>, dim3(bv), dim3(kWalkThreads), 0, s, (const Coef4<T> *)w.c4[1],
                            (const Coef2<T> *)w.c2[1], w.b, a.ny, a.nx, a.VH, (long long)a.pitch);

@@ -96,16 +96,16 @@ struct swh_domain {
     // them): rows per strip of that kernel (0: chosen from its occupancy) and threads
     // per workgroup
     int two_step = 1, rows2 = 0, block2 = 256;
-    // partial sums of the boundary-flux line workgroups of the step launches (12
-    // doubles per workgroup, room for bf_cap of them)
+    // partial sums of the boundary-flux line workgroups of the step launches
+    // (2 kFusedSteps doubles per workgroup, room for bf_cap of them)
     double *d_bfpart = nullptr;
     int bf_cap = 0;
-    // fused launches of several steps: UH/VH on the boundary-flux lines, two buffers of 6
-    // levels x 4 sides x lb_len in turn (d_lb); lb_pending levels of buffer lb_cur, whose steps
+    // fused launches of several steps: UH/VH on the boundary-flux lines, two buffers of
+    // kFusedSteps levels x 4 sides x lb_len in turn (d_lb); lb_pending levels of buffer lb_cur, whose steps
     // ended at lb_t, are still to be summed (within a call only: bf_flush ends it)
     void *d_lb = nullptr;
     int lb_len = 0, lb_cur = 0, lb_pending = 0;
-    double lb_t[6] = {}, lb_dt = 0.0;
+    double lb_t[kFusedSteps] = {}, lb_dt = 0.0;
     int *d_gij = nullptr;          // the gauges' (i, j), 0-based
     std::vector<int> h_gij;
     std::map<int, bool> fit_rows;  // whether they fit the fused kernel's lanes, by rows per strip

@@ -284,16 +284,9 @@ __device__ __forceinline__ Cell cell_clamped(const FVArgs<T> &a, int gi, int j, 
     return clip_raw(a, r);
 }
 
-// Workgroup b of the B of a grid goes to XCD b % 8; this gives it a tile of the XCD's own
-// contiguous range, so that tiles that share rows or cache lines meet in one L2: the update reads each row of
-// fluxes for two rows of cells, and a strip of 61 columns ends inside its neighbour's cache
-// lines (60 rk2 steps of 2000 x 1000 in FP64: 19.6 -> 18.3 ms).
-__device__ __forceinline__ unsigned xcd_tile(unsigned b, unsigned B)
-{
-    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
-    return xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
-}
-
+// Tiles go in xcd_tile's order: the update reads each row of fluxes for two rows of cells, and a
+// strip of 61 columns ends inside its neighbour's cache lines (60 rk2 steps of 2000 x 1000 in FP64:
+// 19.6 -> 18.3 ms).
 template <typename T>
 __device__ __forceinline__ void fv_flux_march_body(const FVArgs<T> &a, int rows)
 {

@@ -57,15 +57,16 @@ struct DevScalars {
 // Boundary-flux sums of a leapfrog step taken by extra workgroups of the step launch
 // (swh_bflux.h): the caller asks for 'want' of them (0: none), the launcher places
 // ey = bf_rows() rows of its grid's width ahead of the tiles. part: the workgroups'
-// partial sums, room for 'cap' workgroups of 12 doubles; t_after: the end time of
-// each step of the launch (NaN: from the device time).
+// partial sums, room for 'cap' workgroups of 2 kFusedSteps doubles; t_after: the end time
+// of each step of the launch (NaN: from the device time).
+constexpr int kFusedSteps = 3;   // steps of a fused launch of a single grid
 struct BfLines {
     int want = 0, cap = 0, ey = 0, n_ext = 2;
     const double *dle = nullptr, *dbe = nullptr;
     DevScalars *sc = nullptr;
     double *part = nullptr;
     double dt = 0.0;
-    double t_after[6] = {};
+    double t_after[kFusedSteps] = {};
 };
 // Rows of line workgroups for a launch gx workgroups wide: enough for 'want' of them
 // (at least 4: one per side), within 'cap'; -1 if they do not fit.
@@ -179,12 +180,12 @@ template <typename T, bool KAHAN>
 hipError_t launch_leapfrogn(const LFArgs<T> &a, int coriolis, int friction_mode, int truely_linear,
                             int linear_friction, int nsrc, int block_x, hipStream_t s, int prefetch, int ns);
 
-// ns (3 or 5; FP64: 3) fused steps of a single grid per launch, with max_stage, boundary
+// kFusedSteps fused steps of a single grid per launch, with max_stage, boundary
 // fluxes and (truely-linear 'linear': a.g_n) one gauge sample inside; the boundary-flux sums
 // of the launch's steps are taken by the next launch, or by launch_bf_flush after the last.
 template <typename T, bool KAHAN>
 hipError_t launch_leapfrog_sg(const LFArgs<T> &a, int coriolis, int friction_mode, int truely_linear,
-                              int linear_friction, int ns, hipStream_t s);
+                              int linear_friction, hipStream_t s);
 template <typename T>
 hipError_t launch_bf_flush(const BfLines &b, int nx, int ny, const T *lines, int len_max, int levels, hipStream_t s);
 // Rows per strip of a fused launch of ns steps over n grids of nx * ny: the least time by
@@ -286,7 +287,7 @@ struct DispArgs {
     const double *dbe, *dle;
     T msl, dlon, dlat, td1, td2;
     int cell;                    // 1: cell-centred (finite-volume) form, 0: staggered
-    int compact;                 // W holds one direction's matrices at a time
+    long long second;            // where VH's matrices lie after UH's, in elements; 0: in the same place
     const DevScalars *sc;        // forward time of the extrapolation from sc->time when set
     double t_fwd;                // else this forward time
 };

@@ -59,4 +59,13 @@ __device__ __forceinline__ double lane_west_or(double v, double edge)
     return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
+// The tile of workgroup b of the B of a grid. Workgroups go round the 8 XCDs (each with its own
+// L2) by their linear index; this gives each XCD a contiguous range of the tiles, in order, so
+// that tiles that share rows or cache lines meet in one L2.
+__device__ __forceinline__ unsigned xcd_tile(unsigned b, unsigned B)
+{
+    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
+    return xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+}
+
 }  // namespace swh

@@ -35,10 +35,11 @@ __device__ __forceinline__ void step1_cell(const LFArgs<T> &a, const T *__restri
 // Neighbours come by lane moves, except in FP32 with friction or depths of the moving surface,
 // where the permutes suit better (they leave the vector pipe): us a step at 2048 x 2048 with
 // permutes / moves, FP32 friction 26.5 / 27.6, FP32 moving depths 18.7 / 19.2, truely linear
-// 18.2 / 18.3, FP64 25.7 / 25.0; 400 x 400 FP64 6.2 / 5.9. Row coefficients are vector loads here: through the scalar cache (scalar_load) they
-// are waited for in the row that uses them, or a row ahead take registers; at 1024 x 1024 in
-// FP64 with friction 15.0 / 16.6 / 18.4 us a step as vector loads / scalar / scalar a row ahead.
-// (4096 x 4096, where a wavefront is seldom waited for, is 6 % faster with scalar loads.)
+// 18.2 / 18.3, FP64 25.7 / 25.0; 400 x 400 FP64 6.2 / 5.9. Row coefficients are vector loads
+// here: through the scalar cache (scalar_load) they are waited for in the row that uses them,
+// or a row ahead take registers; at 1024 x 1024 in FP64 with friction 15.0 / 16.6 / 18.4 us a
+// step as vector loads / scalar / scalar a row ahead. (4096 x 4096 is 3-10 % faster with scalar
+// loads.)
 template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool PF>
 __global__ __launch_bounds__(256) void leapfrog2_kernel(LFArgs<T> a)
 {

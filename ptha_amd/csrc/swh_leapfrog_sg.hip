@@ -26,7 +26,7 @@ __global__ __launch_bounds__(256) void bf_flush_kernel(BfLines b, int nx, int ny
 template <typename T>
 hipError_t launch_bf_flush(const BfLines &b, int nx, int ny, const T *lines, int len_max, int levels, hipStream_t s)
 {
-    if (b.want < 4 || b.want > b.cap || levels < 1 || levels > kBfLevels || !b.part || !b.sc) return hipErrorInvalidValue;
+    if (b.want < 4 || b.want > b.cap || levels < 1 || levels > kFusedSteps || !b.part || !b.sc) return hipErrorInvalidValue;
     hipLaunchKernelGGL(bf_flush_kernel<T>, dim3(b.want), dim3(256), 0, s, b, nx, ny, lines, len_max, levels);
     return hipGetLastError();
 }
@@ -99,21 +99,19 @@ static hipError_t sg_cf(const LFArgs<T> &a, int fric, int tl, int linf, hipStrea
 
 template <typename T, bool KAHAN>
 hipError_t launch_leapfrog_sg(const LFArgs<T> &a, int coriolis, int friction_mode, int truely_linear,
-                              int linear_friction, int ns, hipStream_t s)
+                              int linear_friction, hipStream_t s)
 {
     if (friction_mode > 1 || a.bc_mask || a.src_stride != 0 || a.src_base || (long long)a.pitch * a.ny >= (1LL << 31) ||
         !a.lb_out || a.nx <= 2 * a.bf.n_ext || a.ny <= 2 * a.bf.n_ext || a.lb_len < a.nx - 2 * a.bf.n_ext ||
-        a.lb_len < a.ny - 2 * a.bf.n_ext || (a.mx_levels && (!a.mx || a.mx_levels != (1 << ns) - 1)) ||
-        (a.bf.want && (!a.lb_in || a.lb_levels < 1 || a.lb_levels > kBfLevels || !a.bf.part || !a.bf.sc)))
+        a.lb_len < a.ny - 2 * a.bf.n_ext || (a.mx_levels && (!a.mx || a.mx_levels != (1 << kFusedSteps) - 1)) ||
+        (a.bf.want && (!a.lb_in || a.lb_levels < 1 || a.lb_levels > kFusedSteps || !a.bf.part || !a.bf.sc)))
         return hipErrorInvalidValue;
     const int linf = (friction_mode == 0) && linear_friction;
-    if (ns == 3)
-        return coriolis ? sg_cf<T, KAHAN, true, 3>(a, friction_mode, truely_linear, linf, s)
-                        : sg_cf<T, KAHAN, false, 3>(a, friction_mode, truely_linear, linf, s);
-    return hipErrorInvalidValue;
+    return coriolis ? sg_cf<T, KAHAN, true, kFusedSteps>(a, friction_mode, truely_linear, linf, s)
+                    : sg_cf<T, KAHAN, false, kFusedSteps>(a, friction_mode, truely_linear, linf, s);
 }
 
-template hipError_t launch_leapfrog_sg<double, false>(const LFArgs<double> &, int, int, int, int, int, hipStream_t);
-template hipError_t launch_leapfrog_sg<float, true>(const LFArgs<float> &, int, int, int, int, int, hipStream_t);
+template hipError_t launch_leapfrog_sg<double, false>(const LFArgs<double> &, int, int, int, int, hipStream_t);
+template hipError_t launch_leapfrog_sg<float, true>(const LFArgs<float> &, int, int, int, int, hipStream_t);
 
 }  // namespace swh

@@ -89,17 +89,15 @@ __device__ __forceinline__ T tl_face_depth(T e_near, T e_far, T msl)
 }
 
 // UH at (ii + 1/2, j) from the new stage of cells ii, ii+1 and the pre-step VH of
-// rows j-1 (vhm0, vhm1 at ii, ii+1) and j (vh0, vh1). HPRE (truely linear only): e0
-// carries the face depth h_iph itself (tl_face_depth of the two elevations), e1 unused.
-template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool HPRE = false>
+// rows j-1 (vhm0, vhm1 at ii, ii+1) and j (vh0, vh1).
+template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF>
 __device__ __forceinline__ T mom_u(const LFArgs<T> &a, bool valid, T cu, T fu, T dle_ip1, T fwu, T uh_old, T s0,
                                    T c0, T s1, T c1, T e0, T e1, T vhm0, T vhm1, T vh0, T vh1)
 {
-    static_assert(TL || !HPRE, "precomputed face depths are for the truely-linear scheme");
     const T MIN = T(kMinDepth), HALF = T(0.5), msl = a.msl;
     T h_iph, wet_iph;
     if (TL) {
-        h_iph = HPRE ? e0 : tl_face_depth(e0, e1, msl);
+        h_iph = tl_face_depth(e0, e1, msl);
         wet_iph = T(1);
     } else {
         h_iph = (s0 - e0 > MIN && s1 - e1 > MIN) ? HALF * ((s1 + s0) - (e1 + e0)) : T(0);
@@ -126,17 +124,15 @@ __device__ __forceinline__ T mom_u(const LFArgs<T> &a, bool valid, T cu, T fu, T
 }
 
 // VH at (ii, j + 1/2) from the new stage of rows j, j+1 and the pre-step UH of
-// row j (uh_i at ii, uh_im1 at ii-1) and row j+1 (uhu_i, uhu_im1). HPRE: e0 carries
-// h_jph itself, eu unused.
-template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF, bool HPRE = false>
+// row j (uh_i at ii, uh_im1 at ii-1) and row j+1 (uhu_i, uhu_im1).
+template <typename T, bool KAHAN, bool COR, int FRIC, bool TL, bool LINF>
 __device__ __forceinline__ T mom_v(const LFArgs<T> &a, bool valid, T cv, T fv, T dbe_hi, T fwv, T vh_old, T s0, T c0,
                                    T sup, T cup, T e0, T eu, T uh_i, T uh_im1, T uhu_i, T uhu_im1)
 {
-    static_assert(TL || !HPRE, "precomputed face depths are for the truely-linear scheme");
     const T MIN = T(kMinDepth), HALF = T(0.5), msl = a.msl;
     T h_jph, wet_jph;
     if (TL) {
-        h_jph = HPRE ? e0 : tl_face_depth(e0, eu, msl);
+        h_jph = tl_face_depth(e0, eu, msl);
         wet_jph = T(1);
     } else {
         h_jph = (sup - eu > MIN && s0 - e0 > MIN) ? HALF * ((sup + s0) - (eu + e0)) : T(0);
@@ -179,8 +175,7 @@ __device__ __forceinline__ void lf2_tile(int order, int group, int ey, int &bx, 
     const unsigned gx = gridDim.x, gy = gridDim.y - ey, gz = gridDim.z;
     const unsigned B = gx * gy * gz;
     const unsigned b = blockIdx.x + gx * ((blockIdx.y - ey) + gy * blockIdx.z);
-    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
-    const unsigned L = xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+    const unsigned L = xcd_tile(b, B);
     const unsigned G = (unsigned)group;
     const unsigned gi = L / (gx * gy * G);                 // source group
     const unsigned within = L - gi * (gx * gy * G);

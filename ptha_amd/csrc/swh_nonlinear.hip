@@ -263,15 +263,11 @@ __device__ __forceinline__ NLCell<T> nl_cell(const NLRaw<T> &w, int r, int ny)
     return c;
 }
 
-// This workgroup's tile (column block bx, row or strip by): workgroup b goes to XCD b % 8, and
-// each XCD gets a contiguous range of the tiles, so that those that share rows or cache lines
-// meet in one L2 (80 steps of 1537 x 1021 in FP64: 9.3 -> 8.75 ms; the momentum update reads
-// three rows of fluxes and state).
+// This workgroup's tile (column block bx, row or strip by), in xcd_tile's order: the momentum
+// update reads three rows of fluxes and state (80 steps of 1537 x 1021 in FP64: 9.3 -> 8.75 ms).
 __device__ __forceinline__ void nl_tile(int &bx, int &by)
 {
-    const unsigned gx = gridDim.x, B = gx * gridDim.y, b = blockIdx.x + gx * blockIdx.y;
-    const unsigned xcd = b % 8u, slot = b / 8u, n8 = B / 8u, rem = B % 8u;
-    const unsigned t = xcd < rem ? xcd * (n8 + 1u) + slot : rem * (n8 + 1u) + (xcd - rem) * n8 + slot;
+    const unsigned gx = gridDim.x, t = xcd_tile(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
     by = (int)(t / gx);
     bx = (int)(t - (unsigned)by * gx);
 }
