@@ -27,7 +27,6 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Gcell-updates/s/GPU FP32-comp vs FP64 leapfrog; % HBM peak; unit-sources/hr"
 HBM_PEAK_GBS = 8000.0
-MFMA_FP64_TFLOPS = 78.6   # MI355X dense FP64 matrix peak
 # Algorithmic HBM bytes per cell-update of the fused batched leapfrog step (one read
 # and one write of stage, Kahan term, uh, vh per source; elevation shared):
 BYTES_PER_CELL = {"fp32k": 32.0, "fp64": 48.0}
@@ -155,7 +154,7 @@ def read_traffic(name):
     return {}
 
 
-def roofline(r):
+def roofline(r, shape):
     """The HBM roofline of the batched step kernel. A fused launch advances each of its
     sources by several steps while reading and writing their state (stage, Kahan term,
     UH, VH) once, so its compulsory traffic is 32 B per cell per launch and source (the
@@ -163,12 +162,14 @@ def roofline(r):
     summed over the timed region's launches, over the region's device time (HIP events);
     'per_step_equivalent_gbs' counts 32 B per cell-update instead (what a kernel taking
     one step per pass would have to move), which exceeds the peak when launches fuse
-    steps. 'traffic' is the measured HBM bytes of one full launch (rocprofv3 FETCH_SIZE and
-    WRITE_SIZE scaled by a plain copy kernel) and 'achieved_measured' scales 'achieved' by
-    its ratio to that launch's compulsory bytes. 'valu_issue_frac' is the same launch's
-    VALU wave-instructions over 256 CUs x its busy cycles (one wave-instruction per CU
-    per cycle)."""
+    steps. 'traffic' is the HBM bytes of one full launch in the committed counter profile
+    (rocprofv3 FETCH_SIZE and WRITE_SIZE scaled by a plain copy kernel) and 'achieved_measured'
+    scales 'achieved' by its ratio to that launch's compulsory bytes. 'valu_issue_frac' is
+    the same launch's VALU wave-instructions over 256 CUs x its busy cycles, over the rate of an
+    FMA probe. They are left out where this run's launch shape is not the profile's."""
     t = read_traffic("leapfrog_batch_fp32k")
+    if list(shape) != t.get("launch"):
+        t = {}
     bpc = BYTES_PER_CELL["fp32k"]
     out = {"bound": "hbm", "achieved": round(r["comp_gbs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": round(r["comp_gbs"] / HBM_PEAK_GBS, 4), "traffic": t.get("bytes_per_launch"),
@@ -249,8 +250,8 @@ def secondary_legs(steps):
     m = build_metrics(ca["nx"], ca["ny"], ca["lw"], ca["ll"], True)
     dt = linear_timestep(ca["elev"], m)
     # compulsory bytes per cell and launch: read S, (C,) UH, VH, E, write S, (C,) UH, VH;
-    # swh_evolve_steps takes two steps per launch, so per cell-update half of that
-    for prec, bpc in (("fp32k", 36.0 / 2), ("fp64", 56.0 / 2)):
+    # swh_evolve_steps takes three steps per launch, so per cell-update a third of that
+    for prec, bpc in (("fp32k", 36.0 / 3), ("fp64", 56.0 / 3)):
         d = Domain(ca["nx"], ca["ny"], ca["lw"], ca["ll"], "linear", precision=prec, spherical=True,
                    max_U_variables=())
         U = np.zeros((4, ca["ny"], ca["nx"]))
@@ -264,8 +265,8 @@ def secondary_legs(steps):
         wall = time.perf_counter() - t0
         g = ca["nx"] * ca["ny"] * steps / wall / 1e9
         out["linear_2048sq_" + prec] = dict(gcell_per_s=round(g, 3), ms_per_step=round(1e3 * wall / steps, 4),
-                                            hbm_frac=round(g * bpc / HBM_PEAK_GBS, 4), steps_per_launch=2,
-                                            bytes_per_cell_update=bpc)
+                                            hbm_frac=round(g * bpc / HBM_PEAK_GBS, 4), steps_per_launch=3,
+                                            bytes_per_cell_update=round(bpc, 3))
         d.close()
     # the nonlinear leapfrog on the same grid (Manning 0.025, a 1 m hump), stationary CFL step
     X, Y = np.meshgrid(ca["x"], ca["y"])
@@ -319,11 +320,10 @@ def secondary_legs(steps):
 
 
 def superpose_leg(b, nsrc, max_samples, n_events=4096, seed=20261203):
-    """Earthquake events from the finished batch's gauge series on the FP64 matrix
-    cores: rupture patches of 1-8 x 1-16 unit sources of the 32 x 16 lattice
-    (uniform slip, then stochastic slip), summarised as the maximum stage per gauge;
-    and 64 events as whole series. FLOP/s counts the dense product the kernel does
-    (2 x events x sources (padded to 4) x columns), against the FP64 MFMA peak."""
+    """Earthquake events from the finished batch's gauge series: rupture patches of 1-8 x
+    1-16 unit sources of the 32 x 16 lattice (uniform slip, then stochastic slip),
+    summarised as the maximum stage per gauge; and 64 events as whole series. A term is
+    one source's value added into one event's column."""
     rng = np.random.default_rng(seed)
     nxs, nys = 32, max(1, nsrc // 32)
     events, weights = [], []
@@ -335,19 +335,17 @@ def superpose_leg(b, nsrc, max_samples, n_events=4096, seed=20261203):
         weights.append(rng.lognormal(0.0, 0.5, size=len(src)))
     slip = rng.uniform(0.5, 10.0, size=n_events)
     ng = b._ng
-    kpad = (nsrc + 3) // 4 * 4
+    named = float(sum(len(e) for e in events))
     out = {}
     for name, kw in (("uniform", dict(slip=slip)), ("stochastic", dict(weights=weights))):
         b.superpose(events[:64], summary="max_stage", **{k: v[:64] for k, v in kw.items()})
         _, nv, ms = b.superpose(events, summary="max_stage", timed=True, **kw)
-        flops = 2.0 * n_events * kpad * float(nv.max()) * ng
         out["max_stage_" + name] = dict(events=n_events, kernel_ms=round(ms, 3),
                                         events_per_s=round(n_events / (ms * 1e-3), 1),
-                                        dense_tflops=round(flops / (ms * 1e-3) / 1e12, 2),
-                                        mfma_fp64_frac=round(flops / (ms * 1e-3) / 1e12 / MFMA_FP64_TFLOPS, 4))
+                                        gterms_per_s=round(named * float(nv.max()) * ng / (ms * 1e-3) / 1e9, 2))
     _, nv, ms = b.superpose(events[:64], slip=slip[:64], summary="series", timed=True)
-    flops = 2.0 * 64 * kpad * float(max_samples) * 3 * ng
-    out["series_64_events"] = dict(kernel_ms=round(ms, 3), dense_tflops=round(flops / (ms * 1e-3) / 1e12, 2))
+    terms = float(sum(len(e) for e in events[:64])) * max_samples * 3 * ng
+    out["series_64_events"] = dict(kernel_ms=round(ms, 3), gterms_per_s=round(terms / (ms * 1e-3) / 1e9, 2))
     out["_events"] = (events[:64], slip[:64])
     log("superpose", out)
     return out
@@ -621,7 +619,7 @@ def main():
                                "'linear' leapfrog grid (Coriolis), FP32 state + Kahan-compensated stage" % nsrc,
                    "nx": nx, "ny": ny, "sources": nsrc, "dt_s": dt, "gauges": 64, "gauge_write_s": cfg["gauge_interval"],
                    "launch_fp32k": list(tuned["fp32k"])},
-        "roofline": roofline(r32),
+        "roofline": roofline(r32, tuned["fp32k"]),
         "cpu_baseline": cpu,
     }
     if "fp64" in res:

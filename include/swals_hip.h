@@ -299,10 +299,11 @@ int swh_adjoint_run_schedule(swh_domain *h, double dt, int32_t nsteps, int32_t n
 
 /* Launch shape of the leapfrog step kernel (see swh_batch_set_launch). */
 int swh_domain_set_launch(swh_domain *h, int32_t block_x, int32_t rows_per_block, int32_t variant);
-/* Launch shape of the two-step leapfrog kernel of swh_evolve_steps: threads per
- * workgroup (64..256, a multiple of 64) and rows per strip (4..4096, or 0: chosen from
- * the kernel's occupancy, the default). Results do not depend on it. No counterpart in
- * the reference (a tuning knob of this backend). */
+/* Launch shape of the two-step leapfrog kernel of swh_evolve_steps, which takes the steps
+ * that its launches of three leave: threads per workgroup (64..256, a multiple of 64) and
+ * rows per strip (4..4096, or 0: chosen from the kernel's occupancy, the default). A row
+ * count also makes every step that can run in a pair do so (no launches of three). Results do
+ * not depend on it. No counterpart in the reference (a tuning knob of this backend). */
 int swh_domain_set_launch2(swh_domain *h, int32_t block_x, int32_t rows_per_block);
 
 /* ---- Batched unit sources on one shared grid ----
@@ -359,8 +360,9 @@ int swh_batch_launch_counts(swh_batch *b, int64_t *launches, int64_t *source_lau
  * state traffic, 8 = (batches) consecutive workgroups walk the sources of one tile,
  * 16 = (batches) two fused steps per launch wherever no gauge sample falls between
  * them (friction modes without per-step friction work only), 32 = (single grids)
- * one step per launch in swh_evolve_steps (by default pairs of steps run as one
- * two-step launch where no stage boundary, nesting or max_U update falls between),
+ * one step per launch in swh_evolve_steps (by default runs of steps go three to a launch,
+ * max_stage inside, and others in pairs, where no stage boundary, nesting or other max_U
+ * update falls between),
  * 64 = (batches, two-step launches) XCD-aware tile order: each of the 8 XCDs walks a
  * contiguous range of tiles, columns fastest, then the sources of a group of
  * 2^((variant >> 7) & 7) sources, then strips, so neighbouring tiles, the sources of a

@@ -233,7 +233,8 @@ class Domain:
 
     def set_launch2(self, block_x=256, rows_per_block=0):
         """Launch shape of the two-step leapfrog kernel of evolve_steps (results do not
-        depend on it); rows_per_block 0: chosen from the kernel's occupancy."""
+        depend on it); rows_per_block 0: chosen from the kernel's occupancy, else also no launches
+        of three steps."""
         B.check(self._lib.swh_domain_set_launch2(self._h, int(block_x), int(rows_per_block)),
                 "swh_domain_set_launch2")
 
